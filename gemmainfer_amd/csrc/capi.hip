@@ -271,10 +271,15 @@ size_t gi_w4a16_workspace_bytes(int M, int K, int N, int group_size) {
 int gi_w4a16_linear(const void* A, int a_dtype, const int32_t* B_packed, const void* scales,
                     int n_groups, void* C, int M, int K, int N, int group_size, float softcap,
                     void* workspace, size_t workspace_bytes, void* stream) {
+  int st = GI_OK;
+  if (a_dtype == GI_DTYPE_FP16 &&
+      gi::launch_w4a16_gemm_f16(A, B_packed, scales, n_groups, C, M, K, N, group_size, softcap, workspace,
+                                workspace_bytes, as_stream(stream), &st))
+    return st;
   if (a_dtype == GI_DTYPE_FP16 || a_dtype == GI_DTYPE_FP32)
     return gi::launch_w4a16_generic(A, a_dtype, B_packed, scales, n_groups, C, M, K, N, group_size, softcap,
                                     as_stream(stream));
-  int st = check_bf16_x(a_dtype, "w4a16_linear");
+  st = check_bf16_x(a_dtype, "w4a16_linear");
   if (st != GI_OK) return st;
   return gi::launch_w4a16(A, B_packed, scales, n_groups, C, M, K, N, group_size, softcap,
                           workspace, workspace_bytes, as_stream(stream));

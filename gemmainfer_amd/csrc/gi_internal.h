@@ -109,6 +109,27 @@ int launch_w4a16(const void* A, const int32_t* B, const void* scales, int n_grou
                  int M, int K, int N, int gs, float softcap, void* workspace,
                  size_t workspace_bytes, hipStream_t stream);
 
+// Matrix-core GEMM for more than kGemmMinRows rows (w4a16_gemm.hip), bf16 and
+// fp16.  Its workspace starts behind the arrival counters of the split-K
+// linears (kGemmWsOffset): those stay zero between calls of any shape.
+constexpr int kGemmMinRows = 16;
+constexpr int kMaxGemmSegs = 4;
+constexpr size_t kGemmWsOffset = 16384 * sizeof(int);
+struct GemmSeg {
+  const int32_t* B;   // [K/8, N]
+  const uint16_t* S;  // [G, N]
+  uint16_t* C;        // [M, N]
+  int N, G, tile0;
+};
+bool gemm_supported(int M, int K, int gs, const int* N, int n);
+size_t gemm_workspace_bytes(int M, int K, int gs, const int* N, int n, bool gated);
+int launch_gemm(const void* A, bool f16, int M, int K, int gs, float cap, const GemmSeg* segs, int nseg, bool gated,
+                void* workspace, hipStream_t stream);
+
+bool launch_w4a16_gemm_f16(const void* A, const int32_t* B, const void* scales, int n_groups, void* C, int M, int K,
+                           int N, int gs, float softcap, void* workspace, size_t workspace_bytes, hipStream_t stream,
+                           int* status);
+
 int launch_w4a16_multi(const void* A, int n, const int32_t* const* B, const void* const* scales, const int* n_groups,
                        void* const* C, const int* N, int M, int K, int gs, void* workspace, size_t workspace_bytes,
                        hipStream_t stream);

@@ -856,6 +856,7 @@ inline size_t round_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 // another call's partials breaks the last-arriver test): it is sized for
 // N <= 64 * 16384.
 constexpr size_t kCtrBytes = 16384 * sizeof(int);
+static_assert(kGemmWsOffset >= kCtrBytes, "the GEMM's workspace leaves the arrival counters alone");
 constexpr int kMnWaves = 8;
 constexpr int kMnThreads = kMnWaves * kWave;
 constexpr int kMnCols = 64;
@@ -1254,7 +1255,18 @@ size_t w4a16_workspace_bytes(int M, int K, int N, int gs) {
     return mn_workspace_bytes(M, K, (N + kMnCols - 1) / kMnCols, gs, false);
   // the matrix-core path needs none (scales with the full ceil(K / gs) groups)
   if (gs > 0 && mfma_path(M, K, N, gs, (K + gs - 1) / gs)) return 0;
+  if (gemm_supported(M, K, gs, &N, 1)) return gemm_workspace_bytes(M, K, gs, &N, 1, false);
   return make_plan(M, K, N).total;
+}
+
+// Whether a call of more than 16 rows takes the matrix-core GEMM: its shape
+// and a workspace of the queried size (a smaller one that the VALU path can
+// work with is still served there).
+static bool gemm_ready(int M, int K, int gs, const int* N, int n, bool gated, const void* workspace,
+                       size_t workspace_bytes) {
+  if (!gemm_supported(M, K, gs, N, n)) return false;
+  const size_t need = gemm_workspace_bytes(M, K, gs, N, n, gated);
+  return need == 0 || (workspace && ((uintptr_t)workspace) % kAlign == 0 && workspace_bytes >= need);
 }
 
 int launch_w4a16(const void* A, const int32_t* B, const void* scales, int n_groups, void* C,
@@ -1306,6 +1318,10 @@ int launch_w4a16(const void* A, const int32_t* B, const void* scales, int n_grou
   if (narrow_path(M, K, N)) {
     NarrowSeg sg{B, (const uint16_t*)scales, (uint16_t*)C, N, n_groups, 0};
     return launch_narrow(A, M, K, gs, softcap, &sg, 1, false, stream);
+  }
+  if (gemm_ready(M, K, gs, &N, 1, false, workspace, workspace_bytes)) {
+    const GemmSeg sg{B, (const uint16_t*)scales, (uint16_t*)C, N, n_groups, 0};
+    return launch_gemm(A, false, M, K, gs, softcap, &sg, 1, false, workspace, stream);
   }
   const Plan p = make_plan(M, K, N);
   if (p.ks > 1 && (size_t)p.tiles * sizeof(int) > kCtrBytes)
@@ -1362,6 +1378,19 @@ int launch_w4a16(const void* A, const int32_t* B, const void* scales, int n_grou
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "w4a16 launch");
   return GI_OK;
+}
+
+// fp16 rows past the decode sizes on the same GEMM; false: the caller's VALU
+// kernel, which needs neither the workspace nor the alignment.
+bool launch_w4a16_gemm_f16(const void* A, const int32_t* B, const void* scales, int n_groups, void* C, int M, int K,
+                           int N, int gs, float softcap, void* workspace, size_t workspace_bytes, hipStream_t stream,
+                           int* status) {
+  if (!A || !B || !scales || !C || n_groups <= 0 || N <= 0 || K <= 0) return false;
+  if ((((uintptr_t)A) | ((uintptr_t)B)) % 16 || ((uintptr_t)scales) % 8) return false;
+  if (!gemm_ready(M, K, gs, &N, 1, false, workspace, workspace_bytes)) return false;
+  const GemmSeg sg{B, (const uint16_t*)scales, (uint16_t*)C, N, n_groups, 0};
+  *status = launch_gemm(A, true, M, K, gs, softcap, &sg, 1, false, workspace, stream);
+  return true;
 }
 
 // ---- several projections of one input, and the gated MLP --------------------
@@ -1430,6 +1459,11 @@ int launch_w4a16_multi(const void* A, int n, const int32_t* const* B, const void
   if (narrow_multi(M, K, N, n)) return launch_narrow(A, M, K, gs, 0.f, sg, n, false, stream);
   if (mfma_multi(M, K, N, n, gs))
     return launch_mfma_narrow(A, M, K, gs, 0.f, sg, n, false, workspace, workspace_bytes, stream);
+  if (gemm_ready(M, K, gs, N, n, false, workspace, workspace_bytes)) {
+    GemmSeg gsg[kMaxSegs];
+    for (int i = 0; i < n; ++i) gsg[i] = GemmSeg{sg[i].B, sg[i].S, sg[i].C, N[i], n_groups[i], 0};
+    return launch_gemm(A, false, M, K, gs, 0.f, gsg, n, false, workspace, stream);
+  }
   for (int i = 0; i < n; ++i) {
     const int st = launch_w4a16(A, B[i], scales[i], n_groups[i], C[i], M, K, N[i], gs, 0.f, workspace,
                                 workspace_bytes, stream);
@@ -1442,6 +1476,7 @@ size_t w4a16_multi_workspace_bytes(int n, const int* N, int M, int K, int gs) {
   if (n <= 0 || n > kMaxSegs || !N || M <= 0 || K <= 0) return 0;
   if (narrow_multi(M, K, N, n)) return 0;
   if (gs > 0 && mfma_multi(M, K, N, n, gs)) return mn_workspace_bytes(M, K, mn_tiles(N, n), gs, false);
+  if (gemm_supported(M, K, gs, N, n)) return gemm_workspace_bytes(M, K, gs, N, n, false);
   size_t b = 0;
   for (int i = 0; i < n; ++i) {
     const size_t x = w4a16_workspace_bytes(M, K, N[i], gs);
@@ -1454,6 +1489,8 @@ size_t w4a16_gated_workspace_bytes(int M, int K, int N, int gs) {
   if (M <= 0 || K <= 0 || N <= 0) return 0;
   if (gated_narrow(M, K, N)) return 0;
   if (gs > 0 && gated_mfma(M, K, N, gs)) return mn_workspace_bytes(M, K, (N + kMnCols - 1) / kMnCols, gs, true);
+  const int n2[2] = {N, N};
+  if (gemm_supported(M, K, gs, n2, 2)) return gemm_workspace_bytes(M, K, gs, n2, 2, true);
   return gated_tmp_off(M, K, N) + 2 * round_up((size_t)M * N * 2);
 }
 
@@ -1470,6 +1507,12 @@ int launch_w4a16_gated(const void* A, const int32_t* gB, const void* gS, int gG,
   if (gated_narrow(M, K, N)) return launch_narrow(A, M, K, gs, 0.f, sg, 2, true, stream);
   if (gated_mfma(M, K, N, gs))
     return launch_mfma_narrow(A, M, K, gs, 0.f, sg, 2, true, workspace, workspace_bytes, stream);
+  const int n2[2] = {N, N};
+  if (gemm_ready(M, K, gs, n2, 2, true, workspace, workspace_bytes)) {
+    const GemmSeg gsg[2] = {GemmSeg{gB, (const uint16_t*)gS, (uint16_t*)out, N, gG, 0},
+                            GemmSeg{uB, (const uint16_t*)uS, nullptr, N, uG, 0}};
+    return launch_gemm(A, false, M, K, gs, 0.f, gsg, 2, true, workspace, stream);
+  }
   const size_t need = w4a16_gated_workspace_bytes(M, K, N, gs);
   if (!workspace || workspace_bytes < need || ((uintptr_t)workspace) % kAlign)
     return fail(GI_ERR_WORKSPACE, "w4a16_gated_mlp: workspace missing, misaligned or smaller than "

@@ -1,0 +1,121 @@
+"""W4A16 linears of more than 16 rows (the matrix-core GEMM) against the float64
+oracle, at the edges of its tiles and of its dispatch."""
+import numpy as np
+import pytest
+import torch
+
+from gemmainfer_amd import _lib as L
+from gemmainfer_amd import ops, synth
+from oracle import moe_oracle as O
+
+from helpers import assert_dtype_close
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _f64(t):
+    return t.float().cpu().numpy().astype(np.float64)
+
+
+def _operands(m, k, n, gs, dtype, seed=0):
+    B, S = synth.linear_weights(k, n, gs, seed=seed)
+    x = synth.activations(m, k, seed=seed)
+    return x.to(dtype).to(DEV), B.to(DEV), S.to(dtype).to(DEV)
+
+
+def _check(y, ref, dtype):
+    assert_dtype_close(y, ref, "bf16" if dtype == torch.bfloat16 else "fp16")
+
+
+# rows: one past 16, the 16-, 32- and 64-row tiles' edges, several row blocks;
+# columns: N = 4 mod 64 and mod 256, one tile; K: 8 mod 32, less than a unit, a
+# last group cut short, one past a chunk; enough tiles for the large kernel
+SHAPES = [(17, 64, 64, 64), (32, 136, 68, 64), (33, 512, 200, 64), (64, 2816, 260, 64), (65, 704, 132, 128),
+          (40, 96, 68, 32), (70, 200, 36, 64), (61, 1000, 300, 192), (16 * 5 + 1, 264, 4, 96), (129, 8200, 64, 64),
+          (1281, 264, 2052, 64), (1300, 520, 2304, 32), (2049, 200, 1284, 128), (640, 2816, 4096, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,k,n,gs", SHAPES)
+def test_gemm_parity(m, k, n, gs, dtype):
+    x, B, S = _operands(m, k, n, gs, dtype, seed=m)
+    y = ops.w4a16_linear(x, B, S, gs)
+    ref = O.w4a16_linear(_f64(x), B.cpu().numpy(), _f64(S), gs)
+    _check(y, ref, dtype)
+    assert torch.equal(y, ops.w4a16_linear(x, B, S, gs))
+
+
+@pytest.mark.parametrize("m", [33, 1100])
+def test_gemm_softcap_and_floor_groups(m):
+    """Softcap epilogue; scales with fewer groups than K spans (the rows past
+    the last group are dropped)."""
+    k, n, gs = 320, 2560, 128
+    x, B, S = _operands(m, k, n, gs, torch.bfloat16, seed=3)
+    S = S[: k // gs].contiguous()
+    y = ops.w4a16_linear(x, B, S, gs, softcap=3.0)
+    kk = (k // gs) * gs
+    ref = O.w4a16_linear(_f64(x)[:, :kk], B[: kk // 8].cpu().numpy(), _f64(S), gs)
+    _check(y, 3.0 * np.tanh(ref / 3.0), torch.bfloat16)
+
+
+@pytest.mark.parametrize("m", [24, 50, 1500])
+def test_gemm_multi_and_gated(m):
+    """Several projections in one grid against the oracle; the gated form keeps the torch statements' roundings."""
+    k, gs = 456, 64
+    x = synth.activations(m, k, seed=m).to(DEV)
+    ws = [tuple(t.to(DEV) for t in synth.linear_weights(k, n, gs, seed=n)) for n in (1092, 256, 4)]
+    for y, (B, S) in zip(ops.w4a16_linear_multi(x, ws, gs), ws):
+        _check(y, O.w4a16_linear(_f64(x), B.cpu().numpy(), _f64(S), gs), torch.bfloat16)
+    gate, up = (tuple(t.to(DEV) for t in synth.linear_weights(k, 1092, gs, seed=s)) for s in (7, 8))
+    g, u = (ops.w4a16_linear(x, *w, gs) for w in (gate, up))
+    want = torch.nn.functional.gelu(g.float(), approximate="tanh").to(torch.bfloat16) * u
+    got = ops.gated_mlp_act(x, gate, up, gs)
+    # the two may sum K in different orders, so the rounding of a gate or up
+    # value may fall the other way: an ulp (at most 2^-7 of the value) of the
+    # gate through gelu's largest slope 1.13, of gelu's own rounding, of the up
+    # value, and of the result
+    g, u, w = g.float(), u.float(), want.float()
+    gel = torch.nn.functional.gelu(g, approximate="tanh")
+    bound = 2.0 ** -7 * ((1.13 * g.abs() + 2 * gel.abs()) * u.abs() + w.abs()) + 1e-6
+    assert torch.all((got.float() - w).abs() <= bound)
+
+
+def test_gemm_output_at_any_element():
+    """An output that starts at an odd element (2-byte aligned only), and a
+    strided one, through the drop-in's write semantics."""
+    for m in (30, 1200):
+        k, n, gs = 264, 2564, 64
+        x, B, S = _operands(m, k, n, gs, torch.bfloat16, seed=1)
+        want = ops.w4a16_linear(x, B, S, gs)
+        flat = torch.zeros(m * n + 3, dtype=torch.bfloat16, device=DEV)
+        C = flat[3:].view(m, n)
+        ops.marlin_w4a16(x, B, S, C, gs)
+        assert torch.equal(C, want) and not flat[:3].any()
+
+
+def test_gemm_rows_with_inf_stay_apart():
+    """A row with an infinity, and padding rows, leave the other rows alone."""
+    for m in (19, 1200):
+        k, n, gs = 256, 2304, 64
+        x, B, S = _operands(m, k, n, gs, torch.bfloat16, seed=2)
+        want = ops.w4a16_linear(x, B, S, gs)
+        x[5, 7] = float("inf")
+        y = ops.w4a16_linear(x, B, S, gs)
+        keep = [i for i in range(m) if i != 5]
+        assert torch.equal(y[keep], want[keep])
+        assert not torch.isfinite(y[5].float()).all()
+
+
+def test_gemm_without_its_workspace():
+    """A caller whose workspace holds less than the query is still served where
+    the general kernel needs none."""
+    m, k, n, gs = 20, 64, 65536 + 64, 64
+    x, B, S = _operands(m, k, n, gs, torch.bfloat16, seed=4)
+    y = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    p = lambda t: t.data_ptr()  # noqa: E731
+    st = L.load().gi_w4a16_linear(p(x), L.DTYPE_BF16, p(B), p(S), S.shape[0], p(y), m, k, n, gs, 0.0, None, 0,
+                                  torch.cuda.current_stream().cuda_stream)
+    assert st == L.GI_OK
+    ref = O.w4a16_linear(_f64(x), B[:, :512].cpu().numpy(), _f64(S[:, :512]), gs)
+    _check(y[:, :512], ref, torch.bfloat16)
