@@ -1167,8 +1167,14 @@ int launch_fused_moe(const MoeHostArgs& h) {
                 "fused MoE: workspace missing or smaller than gi_fused_moe_workspace_bytes()");
   if (((uintptr_t)h.workspace) % kAlign)
     return fail(GI_ERR_WORKSPACE, "fused MoE: workspace must be 256-byte aligned");
+  if (moe_prefill_supported(h)) {
+    const size_t base = prefill_base(h.H, h.I);
+    const WsLayout L = ws_layout(1, h.H, h.I, kTaskCols);
+    return launch_moe_prefill(h, (char*)h.workspace + base, h.workspace_bytes - base,
+                              (int*)((char*)h.workspace + L.ctr) + 4 * kCtrStride);
+  }
   if (h.x_dtype == GI_DTYPE_FP16) {
-    // one fp16 token: the one-token kernel's fp16 variant (split bf16
+    // fp16 rows that the grouped GEMM does not take.  One token: the one-token kernel's fp16 variant (split bf16
     // operands); more rows: the 8-row kernel's fp16 variant (fp16 products on
     // q - 8 operands), one launch per 8 rows (~30 us each at the Gemma shapes,
     // against ~120 us for the VALU kernels' launch of 64 slots)
@@ -1181,12 +1187,6 @@ int launch_fused_moe(const MoeHostArgs& h) {
   if (h.x_dtype != GI_DTYPE_BF16) {
     const size_t base = prefill_base(h.H, h.I);
     return launch_moe_generic(h, h.x_dtype, (char*)h.workspace + base, h.workspace_bytes - base);
-  }
-  if (moe_prefill_supported(h)) {
-    const size_t base = prefill_base(h.H, h.I);
-    const WsLayout L = ws_layout(1, h.H, h.I, kTaskCols);
-    return launch_moe_prefill(h, (char*)h.workspace + base, h.workspace_bytes - base,
-                              (int*)((char*)h.workspace + L.ctr) + 4 * kCtrStride);
   }
   if (moe_decode1_supported(h) || moe_decode_supported(h)) {
     // the same layout as the size query (gi_fused_moe_workspace_bytes)

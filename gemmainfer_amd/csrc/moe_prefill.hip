@@ -24,6 +24,11 @@
 //            one bf16 rounding of the sum (the reference adds bf16 atomics,
 //            marlin.cu:583; the order here is fixed)
 //
+// fp16 rows (with the caller's ids) take the same kernels with fp16 products
+// on q - 8 operands, which need no offset product, and fp16 where bf16 stands
+// above.  At 200 rows of the Gemma shapes, group size 64: 1443 us as launches
+// of 8 rows, which read an expert's words once each, 166 us here.
+//
 // The int4 words enter the products as bf16 16 + q (byte permutes) with one
 // more product against a constant -24 operand per 32-k block for the offset,
 // as in the decode kernel; scales apply per group (y += s * (D + Db)).  Rows
@@ -248,7 +253,7 @@ __device__ __forceinline__ uint4 row_operand(__amdgpu_buffer_rsrc_t r, uint32_t 
 // at K.  The first RT row tiles are multiplied (rows past the expert's pairs
 // are zeros): RT is a compile-time value, so the loop has no branch on the
 // tile count (a branch inside it split the scheduling region: slower).
-template <int kPRing, int GSH, int RT>
+template <int kPRing, int GSH, int RT, bool F16>
 __device__ __forceinline__ void grouped_products(__amdgpu_buffer_rsrc_t rw, uint32_t wbase, uint32_t wstep,
                                                  uint32_t wsoff, __amdgpu_buffer_rsrc_t ra, uint32_t roff_own,
                                                  int KB, int G, const uint2* sc_lds, uint4* aring,
@@ -257,7 +262,7 @@ __device__ __forceinline__ void grouped_products(__amdgpu_buffer_rsrc_t rw, uint
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
   const int lq = lane >> 4, lr = lane & 15;
   const bool loader = wave < RT;
-  const uint32_t mq = q4_magic();
+  const uint32_t mq = moe::q4_magic_t<F16>();
   const f32x4_t zf = {0.f, 0.f, 0.f, 0.f};
   const uint4 bc = make_uint4(moe::kQ4BiasPair, moe::kQ4BiasPair, moe::kQ4BiasPair, moe::kQ4BiasPair);
   auto own = [&](int kb) { return kb < KB ? roff_own : kOob; };
@@ -274,13 +279,13 @@ __device__ __forceinline__ void grouped_products(__amdgpu_buffer_rsrc_t rw, uint
   f32x4_t D[kPRT][4], Db[kPRT];
   auto epilogue = [&](int g) {
     const uint2 sv = g < G ? sc_lds[g * 64 + 16 * wave + lr] : make_uint2(0u, 0u);
-    const float sc[4] = {bf16lo(sv.x), bf16hi(sv.x), bf16lo(sv.y), bf16hi(sv.y)};
+    const float sc[4] = {moe::sc_lo<F16>(sv.x), moe::sc_hi<F16>(sv.x), moe::sc_lo<F16>(sv.y), moe::sc_hi<F16>(sv.y)};
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) y[rt][q][jj] += sc[q] * (D[rt][q][jj] + Db[rt][jj]);
+        for (int jj = 0; jj < 4; ++jj) y[rt][q][jj] += sc[q] * (F16 ? D[rt][q][jj] : D[rt][q][jj] + Db[rt][jj]);
   };
 #pragma unroll
   for (int rt = 0; rt < kPRT; ++rt)
@@ -345,27 +350,27 @@ __device__ __forceinline__ void grouped_products(__amdgpu_buffer_rsrc_t rw, uint
     for (int j = 0; j < kPChunk; ++j) {
       const int kb = c * kPChunk + j;
       const uint4 w = wr[j];
-      const uint4 q0 = moe::q4_operand(w.x, mq), q1 = moe::q4_operand(w.y, mq);
-      const uint4 q2 = moe::q4_operand(w.z, mq), q3 = moe::q4_operand(w.w, mq);
+      const uint4 q0 = moe::q4_operand_t<F16>(w.x, mq), q1 = moe::q4_operand_t<F16>(w.y, mq);
+      const uint4 q2 = moe::q4_operand_t<F16>(w.z, mq), q3 = moe::q4_operand_t<F16>(w.w, mq);
       const bool gstart = j % kKbpg == 0;  // compile-time: a group's first product starts from zero
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
         const uint4 A = abuf(c, j, rt);
-        D[rt][0] = moe::mfma_bf16(A, q0, gstart ? zf : D[rt][0]);
-        D[rt][1] = moe::mfma_bf16(A, q1, gstart ? zf : D[rt][1]);
-        D[rt][2] = moe::mfma_bf16(A, q2, gstart ? zf : D[rt][2]);
-        D[rt][3] = moe::mfma_bf16(A, q3, gstart ? zf : D[rt][3]);
-        Db[rt] = moe::mfma_bf16(A, bc, gstart ? zf : Db[rt]);
+        D[rt][0] = moe::mfma_act<F16>(A, q0, gstart ? zf : D[rt][0]);
+        D[rt][1] = moe::mfma_act<F16>(A, q1, gstart ? zf : D[rt][1]);
+        D[rt][2] = moe::mfma_act<F16>(A, q2, gstart ? zf : D[rt][2]);
+        D[rt][3] = moe::mfma_act<F16>(A, q3, gstart ? zf : D[rt][3]);
+        if constexpr (!F16) Db[rt] = moe::mfma_bf16(A, bc, gstart ? zf : Db[rt]);
       }
       // issue order: the A reads, then each product followed by three VALU
-      // operations (the next word's unpack), so that one wave's unpack runs
+      // operations (the next word's unpack; four in fp16, which subtracts 152), so that one wave's unpack runs
       // under its own products (left to itself the compiler puts the whole
       // unpack first: gate/up 111-113 -> 108 us at M=512)
       __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);  // LDS reads
 #pragma unroll
-      for (int p = 0; p < 5 * RT; ++p) {
+      for (int p = 0; p < (F16 ? 4 : 5) * RT; ++p) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one matrix-core product
-        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // three VALU
+        __builtin_amdgcn_sched_group_barrier(0x002, F16 ? 4 : 3, 0);  // the unpack's VALU
       }
       // a group ends at its last k block or at K (a group that K ends inside
       // is finished there: the next group start, past K, resets D); k blocks
@@ -424,7 +429,7 @@ __device__ __forceinline__ ScaleStage<ColOf> scale_stage(const uint16_t* sc_e, i
 
 // gate/up: workgroup (tile t, expert e) owns gate columns [128t, 128t+128)
 // (waves 0, 1) and the same up columns (waves 2, 3); act = bf16(gelu(g)*u).
-template <int GSH>
+template <int GSH, bool F16>
 __global__ __launch_bounds__(kPThreads, 2) void prefill_gu_kernel(PfArgs a) {
   __shared__ float yb[16][256];   // one row tile's gate | up sums
   __shared__ uint4 aring[2 * kPChunk * kPRT * 64];
@@ -457,7 +462,7 @@ __global__ __launch_bounds__(kPThreads, 2) void prefill_gu_kernel(PfArgs a) {
     f32x4_t y[kPRT][4];
     // (all three row tiles: a second instantiation for passes of at most 32
     // pairs, as in down, made this kernel spill and measured slower)
-    grouped_products<kPRingGu, GSH, kPRT>(rw, glive ? wbase : kOob, wstep, e * a.gu_bytes, rx, roff, a.H >> 5,
+    grouped_products<kPRingGu, GSH, kPRT, F16>(rw, glive ? wbase : kOob, wstep, e * a.gu_bytes, rx, roff, a.H >> 5,
                                           a.Ggu, gsc, aring, y);
 #pragma unroll
     for (int rt = 0; rt < kPRT; ++rt) {
@@ -473,7 +478,7 @@ __global__ __launch_bounds__(kPThreads, 2) void prefill_gu_kernel(PfArgs a) {
         const int ic = 128 * tile + c;
         if (j < n_e && ic < a.I)
           a.act[(size_t)(off_e + j) * a.I + (ic & ~7) + moe::mfma_k_pos(ic & 7)] =
-              f32_to_bf16(gelu_tanh(yb[t][c]) * yb[t][128 + c]);
+              moe::f32_to_act<F16>(gelu_tanh(yb[t][c]) * yb[t][128 + c]);
       }
     }
   }
@@ -481,7 +486,7 @@ __global__ __launch_bounds__(kPThreads, 2) void prefill_gu_kernel(PfArgs a) {
 
 // down: workgroup (unit d, expert e) owns output columns [256d, 256d+256);
 // y fp32 rows of the expert's pairs, at each pair's index.
-template <int GSH>
+template <int GSH, bool F16>
 __global__ __launch_bounds__(kPThreads, 2) void prefill_down_kernel(PfArgs a) {
   __shared__ uint4 aring[2 * kPChunk * kPRT * 64];
   // the pair of each row of a pass, in the chunk buffers once the products
@@ -513,10 +518,10 @@ __global__ __launch_bounds__(kPThreads, 2) void prefill_down_kernel(PfArgs a) {
     // two row tiles when the pass has at most 32 pairs (half the experts at
     // M = 512): a third fewer products and epilogue operations
     if (n_e - base <= 32)
-      grouped_products<kPRingDn, GSH, 2>(rw, live ? wbase : kOob, wstep, e * a.dn_bytes, ra, roff, a.I >> 5,
+      grouped_products<kPRingDn, GSH, 2, F16>(rw, live ? wbase : kOob, wstep, e * a.dn_bytes, ra, roff, a.I >> 5,
                                          a.Gd, dsc, aring, y);
     else
-      grouped_products<kPRingDn, GSH, kPRT>(rw, live ? wbase : kOob, wstep, e * a.dn_bytes, ra, roff, a.I >> 5,
+      grouped_products<kPRingDn, GSH, kPRT, F16>(rw, live ? wbase : kOob, wstep, e * a.dn_bytes, ra, roff, a.I >> 5,
                                             a.Gd, dsc, aring, y);
     lds_barrier();  // every wave's last reads of the chunk buffers are done
     if (tid < 16 * kPRT) prow[tid] = pr;
@@ -537,32 +542,41 @@ __global__ __launch_bounds__(kPThreads, 2) void prefill_down_kernel(PfArgs a) {
 // combine: out[t] (+)= sum over slots, in slot order, of w * y[pair]
 // ---------------------------------------------------------------------------
 // A pair's routing as the combine reads it: whether its id is in [0, E)
-// (other ids are skipped, marlin.cu:288-289) and its weight rounded to bf16
-// (marlin.cu:631-636), from the caller's (or the routed) ids and weights.
+// (other ids are skipped, marlin.cu:288-289) and its weight rounded to the
+// activation dtype (marlin.cu:631-636), from the caller's (or the routed) ids and weights.
 // Its result row is the pair index itself.
 struct PfSlots {
   const void* idx;
   const void* w;
   int idx_is64, w_dtype, E;
 };
+template <bool F16>
+__device__ __forceinline__ float load_weight_as_act(const void* w, int dt, int i) {
+  if constexpr (!F16) return load_weight_as_bf16(w, dt, i);
+  if (dt == GI_DTYPE_FP32) return moe::round_to_act<true>(((const float*)w)[i]);
+  if (dt == GI_DTYPE_FP16) return fp16_to_f32(((const uint16_t*)w)[i]);
+  return moe::round_to_act<true>(bf16_to_f32(((const uint16_t*)w)[i]));
+}
+template <bool F16>
 __device__ __forceinline__ void slot_of(const PfSlots& s, int p, int& ok, float& wv) {
   const int id = load_expert_id(s.idx, s.idx_is64, p);
-  wv = load_weight_as_bf16(s.w, s.w_dtype, p);
+  wv = load_weight_as_act<F16>(s.w, s.w_dtype, p);
   ok = id >= 0 && id < s.E;
 }
 
+template <bool F16>
 __global__ __launch_bounds__(256) void prefill_combine_kernel(const float* y, PfSlots sl, uint16_t* out, int H,
                                                               int top_k, int overwrite) {
   const int t = blockIdx.x;
   for (int c = threadIdx.x * 4; c < H; c += 256 * 4) {
     float4 s = overwrite ? make_float4(0.f, 0.f, 0.f, 0.f)
-                         : make_float4(bf16_to_f32(out[(size_t)t * H + c]), bf16_to_f32(out[(size_t)t * H + c + 1]),
-                                       bf16_to_f32(out[(size_t)t * H + c + 2]), bf16_to_f32(out[(size_t)t * H + c + 3]));
+                         : make_float4(moe::act_to_f32<F16>(out[(size_t)t * H + c]), moe::act_to_f32<F16>(out[(size_t)t * H + c + 1]),
+                                       moe::act_to_f32<F16>(out[(size_t)t * H + c + 2]), moe::act_to_f32<F16>(out[(size_t)t * H + c + 3]));
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int k = 0; k < top_k; ++k) {
       int ok;
       float wv;
-      slot_of(sl, t * top_k + k, ok, wv);
+      slot_of<F16>(sl, t * top_k + k, ok, wv);
       const float4 v = *(const float4*)(y + (size_t)(t * top_k + k) * H + c);
       if (!ok) continue;
       acc.x += wv * v.x;
@@ -574,8 +588,8 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const float* y, Pf
     s.y += acc.y;
     s.z += acc.z;
     s.w += acc.w;
-    const uint32_t lo = (uint32_t)f32_to_bf16(s.x) | ((uint32_t)f32_to_bf16(s.y) << 16);
-    const uint32_t hi = (uint32_t)f32_to_bf16(s.z) | ((uint32_t)f32_to_bf16(s.w) << 16);
+    const uint32_t lo = (uint32_t)moe::f32_to_act<F16>(s.x) | ((uint32_t)moe::f32_to_act<F16>(s.y) << 16);
+    const uint32_t hi = (uint32_t)moe::f32_to_act<F16>(s.z) | ((uint32_t)moe::f32_to_act<F16>(s.w) << 16);
     *(uint2*)(out + (size_t)t * H + c) = make_uint2(lo, hi);
   }
 }
@@ -588,6 +602,7 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const float* y, Pf
 // prefill_combine_kernel.
 constexpr int kCombineSlots = 8;
 constexpr int kCombineChunks = 3;
+template <bool F16>
 __global__ __launch_bounds__(256) void prefill_combine8_kernel(const float* y, PfSlots sl, uint16_t* out, int H,
                                                                int top_k, int overwrite) {
   const int t = blockIdx.x;
@@ -595,7 +610,7 @@ __global__ __launch_bounds__(256) void prefill_combine8_kernel(const float* y, P
   __shared__ float swt[kCombineSlots];
   int okv = 0;
   float wvv = 0.f;
-  if ((int)threadIdx.x < top_k) slot_of(sl, t * top_k + threadIdx.x, okv, wvv);
+  if ((int)threadIdx.x < top_k) slot_of<F16>(sl, t * top_k + threadIdx.x, okv, wvv);
   const __amdgpu_buffer_rsrc_t ro = buffer_rsrc(out + (size_t)t * H, overwrite ? 0u : (uint32_t)H * 2u);
   constexpr int kStep = 256 * 4 * kCombineChunks;
   const int nit = (H + kStep - 1) / kStep;  // the same for every thread (the barrier below)
@@ -638,7 +653,7 @@ __global__ __launch_bounds__(256) void prefill_combine8_kernel(const float* y, P
       const int c = c0 + i * 1024;
       if (c >= H) continue;
       float4 s = overwrite ? make_float4(0.f, 0.f, 0.f, 0.f)
-                           : make_float4(bf16lo(o[i].x), bf16hi(o[i].x), bf16lo(o[i].y), bf16hi(o[i].y));
+                           : make_float4(moe::sc_lo<F16>(o[i].x), moe::sc_hi<F16>(o[i].x), moe::sc_lo<F16>(o[i].y), moe::sc_hi<F16>(o[i].y));
       float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
       for (int k = 0; k < kCombineSlots; ++k) {
@@ -652,8 +667,8 @@ __global__ __launch_bounds__(256) void prefill_combine8_kernel(const float* y, P
       s.y += acc.y;
       s.z += acc.z;
       s.w += acc.w;
-      const uint32_t lo = (uint32_t)f32_to_bf16(s.x) | ((uint32_t)f32_to_bf16(s.y) << 16);
-      const uint32_t hi = (uint32_t)f32_to_bf16(s.z) | ((uint32_t)f32_to_bf16(s.w) << 16);
+      const uint32_t lo = (uint32_t)moe::f32_to_act<F16>(s.x) | ((uint32_t)moe::f32_to_act<F16>(s.y) << 16);
+      const uint32_t hi = (uint32_t)moe::f32_to_act<F16>(s.z) | ((uint32_t)moe::f32_to_act<F16>(s.w) << 16);
       *(uint2*)(out + (size_t)t * H + c) = make_uint2(lo, hi);
     }
   }
@@ -679,6 +694,36 @@ PfLayout pf_layout(int M, int top_k, int H, int I, int E) {
   return l;
 }
 
+template <int GSH, bool F16>
+int launch_products_gs(const MoeHostArgs& h, const PfArgs& k, const PfSlots& sl) {
+  const size_t gl = (size_t)h.Ggu * 64 * sizeof(uint2), dl = (size_t)h.Gd * 64 * sizeof(uint2);
+  const dim3 ggrid((h.I + 127) / 128, h.E), dgrid((h.H + 255) / 256, h.E);
+  hipLaunchKernelGGL((prefill_gu_kernel<GSH, F16>), ggrid, dim3(kPThreads), gl, h.stream, k);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return hip_fail(e, "prefill gate/up launch");
+  hipLaunchKernelGGL((prefill_down_kernel<GSH, F16>), dgrid, dim3(kPThreads), dl, h.stream, k);
+  e = hipGetLastError();
+  if (e != hipSuccess) return hip_fail(e, "prefill down launch");
+  if (h.top_k <= kCombineSlots)
+    hipLaunchKernelGGL(prefill_combine8_kernel<F16>, dim3(h.M), dim3(256), 0, h.stream, k.y, sl, (uint16_t*)h.out, h.H,
+                       h.top_k, h.overwrite);
+  else
+    hipLaunchKernelGGL(prefill_combine_kernel<F16>, dim3(h.M), dim3(256), 0, h.stream, k.y, sl, (uint16_t*)h.out, h.H,
+                       h.top_k, h.overwrite);
+  e = hipGetLastError();
+  return e == hipSuccess ? GI_OK : hip_fail(e, "prefill combine launch");
+}
+
+template <bool F16>
+int launch_products(const MoeHostArgs& h, const PfArgs& k, const PfSlots& sl) {
+  switch (k.gsh) {
+    case 0: return launch_products_gs<0, F16>(h, k, sl);
+    case 1: return launch_products_gs<1, F16>(h, k, sl);
+    case 2: return launch_products_gs<2, F16>(h, k, sl);
+    default: return launch_products_gs<3, F16>(h, k, sl);
+  }
+}
+
 int log2_exact(int v) {
   int s = 0;
   while ((1 << s) < v) ++s;
@@ -689,6 +734,18 @@ int log2_exact(int v) {
 
 bool moe_prefill_supported(const MoeHostArgs& h) {
   if (h.M < kPrefillMinRows) return false;
+  // fp16 rows come with the caller's ids.  Operands that sit off 16 bytes, and
+  // scales that end before K (whose rows the other fp16 kernels drop), stay
+  // on those kernels.
+  if (h.x_dtype == GI_DTYPE_FP16) {
+    if (h.logits) return false;
+    if (((uintptr_t)h.x | (uintptr_t)h.gu_packed | (uintptr_t)h.gu_scales | (uintptr_t)h.d_packed |
+         (uintptr_t)h.d_scales | (uintptr_t)h.out) % 16)
+      return false;
+    if ((long long)h.Ggu * h.gs < h.H || (long long)h.Gd * h.gs < h.I) return false;
+  } else if (h.x_dtype != GI_DTYPE_BF16) {
+    return false;
+  }
   if (h.H % 64 || h.I % 32) return false;
   if (h.gs % 32 || log2_exact(h.gs / 32) < 0 || kPChunk % (h.gs / 32)) return false;
   if (h.top_k > 64 || h.E > 1024) return false;
@@ -783,34 +840,8 @@ int launch_moe_prefill(const MoeHostArgs& h, void* workspace, size_t ws_bytes, i
   k.dn_bytes = (uint32_t)((size_t)(h.I / 8) * h.H * 4);
   k.dn_total = (uint32_t)((size_t)h.E * k.dn_bytes);
   k.act_bytes = (uint32_t)((size_t)P * h.I * 2);
-  const size_t gl = (size_t)h.Ggu * 64 * sizeof(uint2), dl = (size_t)h.Gd * 64 * sizeof(uint2);
-  const dim3 ggrid((h.I + 127) / 128, h.E), dgrid((h.H + 255) / 256, h.E);
-  switch (k.gsh) {
-    case 0: hipLaunchKernelGGL(prefill_gu_kernel<0>, ggrid, dim3(kPThreads), gl, h.stream, k); break;
-    case 1: hipLaunchKernelGGL(prefill_gu_kernel<1>, ggrid, dim3(kPThreads), gl, h.stream, k); break;
-    case 2: hipLaunchKernelGGL(prefill_gu_kernel<2>, ggrid, dim3(kPThreads), gl, h.stream, k); break;
-    default: hipLaunchKernelGGL(prefill_gu_kernel<3>, ggrid, dim3(kPThreads), gl, h.stream, k); break;
-  }
-  e = hipGetLastError();
-  if (e != hipSuccess) return hip_fail(e, "prefill gate/up launch");
-  switch (k.gsh) {
-    case 0: hipLaunchKernelGGL(prefill_down_kernel<0>, dgrid, dim3(kPThreads), dl, h.stream, k); break;
-    case 1: hipLaunchKernelGGL(prefill_down_kernel<1>, dgrid, dim3(kPThreads), dl, h.stream, k); break;
-    case 2: hipLaunchKernelGGL(prefill_down_kernel<2>, dgrid, dim3(kPThreads), dl, h.stream, k); break;
-    default: hipLaunchKernelGGL(prefill_down_kernel<3>, dgrid, dim3(kPThreads), dl, h.stream, k); break;
-  }
-  e = hipGetLastError();
-  if (e != hipSuccess) return hip_fail(e, "prefill down launch");
   const PfSlots sl{f.idx, w, f.idx_is64, w_dtype, h.E};
-  if (h.top_k <= kCombineSlots)
-    hipLaunchKernelGGL(prefill_combine8_kernel, dim3(h.M), dim3(256), 0, h.stream, k.y, sl, (uint16_t*)h.out, h.H,
-                       h.top_k, h.overwrite);
-  else
-    hipLaunchKernelGGL(prefill_combine_kernel, dim3(h.M), dim3(256), 0, h.stream, k.y, sl, (uint16_t*)h.out, h.H,
-                       h.top_k, h.overwrite);
-  e = hipGetLastError();
-  if (e != hipSuccess) return hip_fail(e, "prefill combine launch");
-  return GI_OK;
+  return h.x_dtype == GI_DTYPE_FP16 ? launch_products<true>(h, k, sl) : launch_products<false>(h, k, sl);
 }
 
 }  // namespace gi

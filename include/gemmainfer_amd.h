@@ -114,7 +114,8 @@ int gi_moe_align(const void* idx, int idx_dtype, int M, int top_k, int E,
  *   idx        int32|int64 [M*top_k]  w  bf16|fp16|fp32 [M*top_k]
  *   out        T [M, H]               accumulated into (caller zeroes it)
  * T = x_dtype: bf16, fp16 or fp32 (marlin.cu:694-700).  bf16 runs the paths
- * below; fp16 and fp32 run VALU kernels (fp32 arithmetic, the routing
+ * below, and so does fp16 where operands are 16-byte aligned and the scales
+ * cover K; other fp16 and fp32 calls run VALU kernels (fp32 arithmetic, the routing
  * weights cast to T, the activation stored in T, one rounding of the output
  * in T; the dequantised weights are never rounded; Token-Union in launches
  * of up to 64 slots, top_k <= 64: alignment, gate/up, down, combine).

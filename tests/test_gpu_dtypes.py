@@ -223,6 +223,35 @@ def test_moe_fp16_deterministic_and_multi_launch(m):
     assert_dtype_close(outs[0], _oracle(W, x, idx, w, torch.zeros(m, H), gs, "fp16"), "fp16", f"fp16 m={m}")
 
 
+@pytest.mark.parametrize("h,i,e,k,gs", [(256, 160, 16, 8, 64), (320, 96, 24, 12, 32), (256, 256, 8, 2, 256),
+                                        (512, 128, 300, 4, 128)])
+@pytest.mark.parametrize("m", [64, 101])
+def test_moe_fp16_grouped_gemm(h, i, e, k, gs, m):
+    """fp16 rows on the grouped GEMM: one to three row tiles per expert and
+    more than one pass, a partial column tile and group, both combines,
+    skipped ids and repeated experts, and the same calls with out at 8 bytes
+    past a multiple of 16, which the VALU kernels take."""
+    dt = torch.float16
+    W = _moe_weights(e, h, i, gs, seed=950 + h + i, dt=dt)
+    Wd = {n: v.to(DEV) for n, v in W.items()}
+    g = torch.Generator().manual_seed(951 + m)
+    x = synth.activations(m, h, seed=952 + m).to(dt)
+    x[0, :8] = torch.tensor([6e-8, -6e-8, 1e-6, -3e-5, 0.0, 17.0078125, -1.0009765625, 0.33325195]).to(dt)
+    ids = torch.topk(torch.randn(m, e, generator=g) + 2 * torch.randn(1, e, generator=g), k, dim=-1).indices
+    ids[0, 0], ids[m - 1, 1], ids[1, 0] = -1, e, ids[1, 1]
+    for idx, w in [(ids, torch.rand(m, k, generator=g)),
+                   (ids.to(torch.int32), torch.softmax(torch.randn(m, k, generator=g), -1).to(torch.bfloat16)),
+                   (torch.full((m, k), e - 1, dtype=torch.int32), (torch.rand(m, k, generator=g) / 4).to(dt))]:
+        out_in = (torch.randn(m, h, generator=g) * 0.1).to(dt)
+        ref = _oracle(W, x, idx, w.to(dt), out_in, gs, "fp16")
+        for off in (0, 4):
+            out = torch.empty(m * h + off, dtype=dt, device=DEV)[off:].view(m, h).copy_(out_in)
+            gemmainfer_csrc.fused_batched_moe(x.to(DEV), Wd["gate_up_packed"], Wd["gate_up_scales"],
+                                              Wd["down_packed"], Wd["down_scales"], idx.to(DEV), w.to(DEV), out, gs)
+            torch.cuda.synchronize()
+            assert_dtype_close(out, ref, "fp16", f"fp16 grouped h={h} k={k} gs={gs} m={m} off={off}")
+
+
 @pytest.mark.parametrize("tag", ["fp16", "fp32"])
 def test_moe_duplicates_invalid_ids_and_many_rows(tag):
     dt = DT[tag]
