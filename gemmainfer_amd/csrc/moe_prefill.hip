@@ -15,7 +15,7 @@
 //            matrix-core k order
 //   gate/up  grid (I/128 column tiles, E): 16-token row tiles of the expert's
 //            pairs (A = gathered x rows) times the unpacked int4 words (B),
-//            v_mfma_f32_16x16x32_bf16, 48 pairs per pass; act =
+//            v_mfma_f32_16x16x32_bf16, 48 or 16 pairs per pass; act =
 //            bf16(gelu_tanh(gate) * up) (marlin.cu:414-423)
 //   down     grid (H/256 column units, E): the same over the act rows, fp32
 //            results per pair
@@ -247,17 +247,17 @@ __device__ __forceinline__ uint4 row_operand(__amdgpu_buffer_rsrc_t r, uint32_t 
 // scale * (D + Db).  Weights: rw/wbase (+ kb * wstep), activations: ra with
 // this wave's own row tile offset (waves < kPRT), scales:
 // sc_lds[g * 64 + 16 w + lr] (4 bf16; groups past G scale by zero), aring:
-// two chunk buffers [2][kPChunk][kPRT][64] uint4.  The group size (32 <<
+// two chunk buffers [2][kPChunk][YT][64] uint4 (YT: the kernel's tiles per pass).  The group size (32 <<
 // GSH) is a compile-time value, so every group end inside a chunk is known to
 // the compiler (a chunk holds whole groups); a last partial group is finished
 // at K.  The first RT row tiles are multiplied (rows past the expert's pairs
 // are zeros): RT is a compile-time value, so the loop has no branch on the
 // tile count (a branch inside it split the scheduling region: slower).
-template <int kPRing, int GSH, int RT, bool F16>
+template <int kPRing, int GSH, int RT, bool F16, int YT>
 __device__ __forceinline__ void grouped_products(__amdgpu_buffer_rsrc_t rw, uint32_t wbase, uint32_t wstep,
                                                  uint32_t wsoff, __amdgpu_buffer_rsrc_t ra, uint32_t roff_own,
                                                  int KB, int G, const uint2* sc_lds, uint4* aring,
-                                                 f32x4_t (&y)[kPRT][4]) {
+                                                 f32x4_t (&y)[YT][4]) {
   constexpr int kKbpg = 1 << GSH;
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
   const int lq = lane >> 4, lr = lane & 15;
@@ -276,7 +276,7 @@ __device__ __forceinline__ void grouped_products(__amdgpu_buffer_rsrc_t rw, uint
         __builtin_amdgcn_raw_buffer_load_b128(rw, (wlive && kb < KB) ? wb + (uint32_t)kb * wstep : kOob, 0, 2);
     return make_uint4(v.x, v.y, v.z, v.w);
   };
-  f32x4_t D[kPRT][4], Db[kPRT];
+  f32x4_t D[RT][4], Db[RT];
   auto epilogue = [&](int g) {
     const uint2 sv = g < G ? sc_lds[g * 64 + 16 * wave + lr] : make_uint2(0u, 0u);
     const float sc[4] = {moe::sc_lo<F16>(sv.x), moe::sc_hi<F16>(sv.x), moe::sc_lo<F16>(sv.y), moe::sc_hi<F16>(sv.y)};
@@ -288,11 +288,11 @@ __device__ __forceinline__ void grouped_products(__amdgpu_buffer_rsrc_t rw, uint
         for (int jj = 0; jj < 4; ++jj) y[rt][q][jj] += sc[q] * (F16 ? D[rt][q][jj] : D[rt][q][jj] + Db[rt][jj]);
   };
 #pragma unroll
-  for (int rt = 0; rt < kPRT; ++rt)
+  for (int rt = 0; rt < YT; ++rt)
 #pragma unroll
     for (int q = 0; q < 4; ++q) y[rt][q] = zf;
   static_assert(kPChunk % kKbpg == 0 && kPRing == kPChunk, "chunks hold whole groups; one ring slot per k block");
-  auto abuf = [&](int c, int j, int rt) -> uint4& { return aring[(((c & 1) * kPChunk + j) * kPRT + rt) * 64 + lane]; };
+  auto abuf = [&](int c, int j, int rt) -> uint4& { return aring[(((c & 1) * kPChunk + j) * YT + rt) * 64 + lane]; };
   // A tiles stream through LDS a chunk of kPChunk k blocks at a time (one
   // barrier per chunk): loader wave rt keeps the next chunk of its row tile
   // in registers and writes it into the free chunk buffer.  The chunk loop is
@@ -429,10 +429,19 @@ __device__ __forceinline__ ScaleStage<ColOf> scale_stage(const uint16_t* sc_e, i
 
 // gate/up: workgroup (tile t, expert e) owns gate columns [128t, 128t+128)
 // (waves 0, 1) and the same up columns (waves 2, 3); act = bf16(gelu(g)*u).
-template <int GSH, bool F16>
-__global__ __launch_bounds__(kPThreads, 2) void prefill_gu_kernel(PfArgs a) {
-  __shared__ float yb[16][256];   // one row tile's gate | up sums
-  __shared__ uint4 aring[2 * kPChunk * kPRT * 64];
+//
+// RT row tiles per pass: three where experts have many pairs, one where they
+// have few (pf_row_tiles).  One drops the products with rows of zeros, and
+// with the row tile's sums in the chunk buffers (free by then), a third of the
+// buffers and 168 registers three workgroups fit a CU instead of two: more of
+// the words are in flight, which is what bounds a small batch.  29 rows that
+// choose independently (Gemma shapes, group size 64, bf16): 220.9 us as 8-row
+// launches, 82.4 us here.
+template <int GSH, bool F16, int RT>
+__global__ __launch_bounds__(kPThreads, RT == 1 ? 3 : 2) void prefill_gu_kernel(PfArgs a) {
+  __shared__ uint4 aring[2 * kPChunk * RT * 64 + (RT == 1 ? 0 : 1024)];
+  // one row tile's gate | up sums
+  float (*yb)[256] = reinterpret_cast<float (*)[256]>(RT == 1 ? aring : aring + 2 * kPChunk * RT * 64);
   extern __shared__ uint2 gsc[];  // [Ggu][64]: 4 scales of each column quad
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
   const int lq = lane >> 4, lr = lane & 15;
@@ -454,18 +463,18 @@ __global__ __launch_bounds__(kPThreads, 2) void prefill_gu_kernel(PfArgs a) {
   // a wave whose 64 gate (or up) columns all lie past I (the last tile when
   // I is not a multiple of 128) has no products to run
   const bool glive = 128 * tile + 64 * (wave & 1) < a.I;
-  for (int base = 0; base < n_e; base += 16 * kPRT) {
-    // this wave's row tile (waves < kPRT load the A operands for all)
+  for (int base = 0; base < n_e; base += 16 * RT) {
+    // this wave's row tile (waves < RT load the A operands for all)
     const int jo = base + 16 * wave + lr;
-    const uint32_t roff = wave < kPRT && jo < n_e ? (uint32_t)(a.order[off_e + jo] / a.top_k) * (uint32_t)a.H * 2u
+    const uint32_t roff = wave < RT && jo < n_e ? (uint32_t)(a.order[off_e + jo] / a.top_k) * (uint32_t)a.H * 2u
                                                  : kOob;
-    f32x4_t y[kPRT][4];
-    // (all three row tiles: a second instantiation for passes of at most 32
+    f32x4_t y[RT][4];
+    // (all RT row tiles: a second instantiation for passes of at most 32
     // pairs, as in down, made this kernel spill and measured slower)
-    grouped_products<kPRingGu, GSH, kPRT, F16>(rw, glive ? wbase : kOob, wstep, e * a.gu_bytes, rx, roff, a.H >> 5,
+    grouped_products<kPRingGu, GSH, RT, F16>(rw, glive ? wbase : kOob, wstep, e * a.gu_bytes, rx, roff, a.H >> 5,
                                           a.Ggu, gsc, aring, y);
 #pragma unroll
-    for (int rt = 0; rt < kPRT; ++rt) {
+    for (int rt = 0; rt < RT; ++rt) {
       __syncthreads();
 #pragma unroll
       for (int q = 0; q < 4; ++q)
@@ -486,9 +495,9 @@ __global__ __launch_bounds__(kPThreads, 2) void prefill_gu_kernel(PfArgs a) {
 
 // down: workgroup (unit d, expert e) owns output columns [256d, 256d+256);
 // y fp32 rows of the expert's pairs, at each pair's index.
-template <int GSH, bool F16>
-__global__ __launch_bounds__(kPThreads, 2) void prefill_down_kernel(PfArgs a) {
-  __shared__ uint4 aring[2 * kPChunk * kPRT * 64];
+template <int GSH, bool F16, int RT>
+__global__ __launch_bounds__(kPThreads, RT == 1 ? 3 : 2) void prefill_down_kernel(PfArgs a) {
+  __shared__ uint4 aring[2 * kPChunk * RT * 64];
   // the pair of each row of a pass, in the chunk buffers once the products
   // are done (no LDS beyond theirs: the 160 KB limit check counts them only)
   int* prow = reinterpret_cast<int*>(aring);
@@ -508,26 +517,26 @@ __global__ __launch_bounds__(kPThreads, 2) void prefill_down_kernel(PfArgs a) {
   const __amdgpu_buffer_rsrc_t ra = buffer_rsrc(a.act, a.act_bytes);
   const uint32_t wbase = ((uint32_t)lq * a.H + col) * 4u;
   const uint32_t wstep = (uint32_t)a.H * 16u;
-  for (int base = 0; base < n_e; base += 16 * kPRT) {
+  for (int base = 0; base < n_e; base += 16 * RT) {
     // each row's pair index (its result row): loaded here, written to LDS
     // after the products (the load must not hold the products' first loads)
-    const int pr = tid < 16 * kPRT && base + tid < n_e ? a.order[off_e + base + tid] : 0;
+    const int pr = tid < 16 * RT && base + tid < n_e ? a.order[off_e + base + tid] : 0;
     const int jo = base + 16 * wave + lr;
-    const uint32_t roff = wave < kPRT && jo < n_e ? (uint32_t)(off_e + jo) * (uint32_t)a.I * 2u : kOob;
-    f32x4_t y[kPRT][4];
+    const uint32_t roff = wave < RT && jo < n_e ? (uint32_t)(off_e + jo) * (uint32_t)a.I * 2u : kOob;
+    f32x4_t y[RT][4];
     // two row tiles when the pass has at most 32 pairs (half the experts at
     // M = 512): a third fewer products and epilogue operations
-    if (n_e - base <= 32)
-      grouped_products<kPRingDn, GSH, 2, F16>(rw, live ? wbase : kOob, wstep, e * a.dn_bytes, ra, roff, a.I >> 5,
+    if (RT == 3 && n_e - base <= 32)
+      grouped_products<kPRingDn, GSH, RT == 3 ? 2 : RT, F16>(rw, live ? wbase : kOob, wstep, e * a.dn_bytes, ra, roff, a.I >> 5,
                                          a.Gd, dsc, aring, y);
     else
-      grouped_products<kPRingDn, GSH, kPRT, F16>(rw, live ? wbase : kOob, wstep, e * a.dn_bytes, ra, roff, a.I >> 5,
+      grouped_products<kPRingDn, GSH, RT, F16>(rw, live ? wbase : kOob, wstep, e * a.dn_bytes, ra, roff, a.I >> 5,
                                             a.Gd, dsc, aring, y);
     lds_barrier();  // every wave's last reads of the chunk buffers are done
-    if (tid < 16 * kPRT) prow[tid] = pr;
+    if (tid < 16 * RT) prow[tid] = pr;
     lds_barrier();  // (the next pass's products start with a barrier before they write the buffers)
 #pragma unroll
-    for (int rt = 0; rt < kPRT; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
         const int j = base + 16 * rt + 4 * lq + jj;
@@ -694,14 +703,23 @@ PfLayout pf_layout(int M, int top_k, int H, int I, int E) {
   return l;
 }
 
-template <int GSH, bool F16>
+// Row tiles per pass: one below 64 rows, where most experts have few pairs.
+// Above, tokens that agree on few experts fill three tiles: Gemma shapes,
+// group size 64, bf16, three / one at 64 rows 168.7 / 89.2 us for tokens that
+// choose independently, 118.7 / 143.8 us for ones that agree on most, 80 rows
+// 169.8 / 91.2 and 160.7 / 174.4 us.  (Several workgroups for an expert's
+// passes run those faster, 90 us at 80 rows, but the ones without a pass cost
+// the even case as much as it gains: 512 rows 199 / 282 us.)
+int pf_row_tiles(int M) { return M < 64 ? 1 : kPRT; }
+
+template <int GSH, bool F16, int RT>
 int launch_products_gs(const MoeHostArgs& h, const PfArgs& k, const PfSlots& sl) {
   const size_t gl = (size_t)h.Ggu * 64 * sizeof(uint2), dl = (size_t)h.Gd * 64 * sizeof(uint2);
   const dim3 ggrid((h.I + 127) / 128, h.E), dgrid((h.H + 255) / 256, h.E);
-  hipLaunchKernelGGL((prefill_gu_kernel<GSH, F16>), ggrid, dim3(kPThreads), gl, h.stream, k);
+  hipLaunchKernelGGL((prefill_gu_kernel<GSH, F16, RT>), ggrid, dim3(kPThreads), gl, h.stream, k);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "prefill gate/up launch");
-  hipLaunchKernelGGL((prefill_down_kernel<GSH, F16>), dgrid, dim3(kPThreads), dl, h.stream, k);
+  hipLaunchKernelGGL((prefill_down_kernel<GSH, F16, RT>), dgrid, dim3(kPThreads), dl, h.stream, k);
   e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "prefill down launch");
   if (h.top_k <= kCombineSlots)
@@ -714,13 +732,13 @@ int launch_products_gs(const MoeHostArgs& h, const PfArgs& k, const PfSlots& sl)
   return e == hipSuccess ? GI_OK : hip_fail(e, "prefill combine launch");
 }
 
-template <bool F16>
+template <bool F16, int RT>
 int launch_products(const MoeHostArgs& h, const PfArgs& k, const PfSlots& sl) {
   switch (k.gsh) {
-    case 0: return launch_products_gs<0, F16>(h, k, sl);
-    case 1: return launch_products_gs<1, F16>(h, k, sl);
-    case 2: return launch_products_gs<2, F16>(h, k, sl);
-    default: return launch_products_gs<3, F16>(h, k, sl);
+    case 0: return launch_products_gs<0, F16, RT>(h, k, sl);
+    case 1: return launch_products_gs<1, F16, RT>(h, k, sl);
+    case 2: return launch_products_gs<2, F16, RT>(h, k, sl);
+    default: return launch_products_gs<3, F16, RT>(h, k, sl);
   }
 }
 
@@ -734,17 +752,17 @@ int log2_exact(int v) {
 
 bool moe_prefill_supported(const MoeHostArgs& h) {
   if (h.M < kPrefillMinRows) return false;
-  // fp16 rows come with the caller's ids.  Operands that sit off 16 bytes, and
-  // scales that end before K (whose rows the other fp16 kernels drop), stay
-  // on those kernels.
-  if (h.x_dtype == GI_DTYPE_FP16) {
-    if (h.logits) return false;
+  if (h.x_dtype != GI_DTYPE_BF16 && h.x_dtype != GI_DTYPE_FP16) return false;
+  if (h.x_dtype == GI_DTYPE_FP16 && h.logits) return false;  // fp16 rows come with the caller's ids
+  // fp16 rows, and fewer than 64 of bf16: operands that sit off 16 bytes, and
+  // scales that end before K, stay on the kernels that take launches of rows,
+  // and so does a routing that only their launch refuses
+  if (h.x_dtype == GI_DTYPE_FP16 || h.M < 64) {
     if (((uintptr_t)h.x | (uintptr_t)h.gu_packed | (uintptr_t)h.gu_scales | (uintptr_t)h.d_packed |
          (uintptr_t)h.d_scales | (uintptr_t)h.out) % 16)
       return false;
     if ((long long)h.Ggu * h.gs < h.H || (long long)h.Gd * h.gs < h.I) return false;
-  } else if (h.x_dtype != GI_DTYPE_BF16) {
-    return false;
+    if (h.logits && (h.E > moe::kRouteMaxExperts || h.top_k > h.E)) return false;
   }
   if (h.H % 64 || h.I % 32) return false;
   if (h.gs % 32 || log2_exact(h.gs / 32) < 0 || kPChunk % (h.gs / 32)) return false;
@@ -841,7 +859,9 @@ int launch_moe_prefill(const MoeHostArgs& h, void* workspace, size_t ws_bytes, i
   k.dn_total = (uint32_t)((size_t)h.E * k.dn_bytes);
   k.act_bytes = (uint32_t)((size_t)P * h.I * 2);
   const PfSlots sl{f.idx, w, f.idx_is64, w_dtype, h.E};
-  return h.x_dtype == GI_DTYPE_FP16 ? launch_products<true>(h, k, sl) : launch_products<false>(h, k, sl);
+  const bool f16 = h.x_dtype == GI_DTYPE_FP16;
+  if (pf_row_tiles(h.M) == 1) return f16 ? launch_products<true, 1>(h, k, sl) : launch_products<false, 1>(h, k, sl);
+  return f16 ? launch_products<true, kPRT>(h, k, sl) : launch_products<false, kPRT>(h, k, sl);
 }
 
 }  // namespace gi

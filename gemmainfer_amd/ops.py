@@ -222,7 +222,7 @@ def fused_batched_moe(x, gate_up_packed, gate_up_scales, down_packed, down_scale
 def moe_layer(x, router_logits, gate_up_packed, gate_up_scales, down_packed, down_scales,
               top_k, group_size, expert_scale=None, out=None, *, spin_limit: int = 0):
     """Router tail + fused MoE (gemma.py:77-98): one launch per 8 rows up to
-    63 rows, and from 64 rows the grouped-GEMM prefill path (routing, align,
+    11 rows, and from 12 rows the grouped-GEMM prefill path (routing, align,
     gate/up, down and combine launches).
 
     Returns (out [M, H] bf16 -- overwritten, idx int32 [M, top_k],

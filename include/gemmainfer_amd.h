@@ -120,7 +120,7 @@ int gi_moe_align(const void* idx, int idx_dtype, int M, int top_k, int E,
  * in T; the dequantised weights are never rounded; Token-Union in launches
  * of up to 64 slots, top_k <= 64: alignment, gate/up, down, combine).
  * One kernel launch per 256/top_k rows (8 rows on the decode kernel); from
- * 64 rows with top_k <= 64, a power-of-two multiple of 32 as group size,
+ * 12 rows with top_k <= 64, a power-of-two multiple of 32 as group size,
  * H % 64 == 0 and I % 32 == 0, the grouped-GEMM prefill path (align with
  * the x reorder, gate/up, down, combine launches; each active expert read
  * once).
@@ -180,7 +180,7 @@ int gi_fused_batched_moe_static_status(int32_t* host_status, int clear, void* st
 /* Router + fused MoE: logits [M, E] (bf16/fp32) are routed as
  * gi_moe_route_topk_softmax does (weights rounded to bf16), out[M, H] is
  * OVERWRITTEN with the MoE output, and out_idx/out_w (may be NULL) receive
- * the routing.  Up to 8 rows per launch; from 64 rows (group size a power of
+ * the routing.  Up to 8 rows per launch; from 12 rows (group size a power of
  * two times 32, H % 64 == 0, I % 32 == 0) the sorted-by-expert grouped-GEMM
  * prefill path replaces the 8-row slices of gemma.py:99-112 (routing with
  * the align and the x reorder, gate/up, down, combine launches).           */

@@ -252,6 +252,44 @@ def test_moe_fp16_grouped_gemm(h, i, e, k, gs, m):
             assert_dtype_close(out, ref, "fp16", f"fp16 grouped h={h} k={k} gs={gs} m={m} off={off}")
 
 
+@pytest.mark.parametrize("tag", ["bf16", "fp16"])
+@pytest.mark.parametrize("m", [11, 12, 17, 63, 64, 145])
+def test_moe_grouped_gemm_few_rows(tag, m):
+    """The smallest calls on the grouped GEMM: the last row count of the 8-row
+    launches (11) and the first here, one row tile per pass below 64 rows and
+    three above, an expert's
+    passes (none to more than 15, with every pair on
+    one expert), skipped ids, and the same bits from a second call."""
+    dt = torch.bfloat16 if tag == "bf16" else torch.float16
+    h, i, e, k, gs = 256, 160, 40, 4, 64
+    W = _moe_weights(e, h, i, gs, seed=970, dt=dt)
+    Wd = {n: v.to(DEV) for n, v in W.items()}
+    g = torch.Generator().manual_seed(971 + m)
+    x = synth.activations(m, h, seed=972 + m).to(dt)
+    even = torch.stack([torch.randperm(e, generator=g)[:k] for _ in range(m)]).to(torch.int32)
+    skewed = torch.topk(torch.randn(m, e, generator=g) + 3 * torch.randn(1, e, generator=g), k, dim=-1).indices
+    skewed[0, 1], skewed[m - 1, 0] = e, -1
+    w = (torch.rand(m, k, generator=g) / 4).to(dt)
+    xd, wd = x.to(DEV), w.to(DEV)
+    for idx in (even, skewed, torch.full((m, k), 7, dtype=torch.int32)):
+        idxd = idx.to(DEV)
+        out = torch.zeros(m, h, dtype=dt, device=DEV)
+
+        def call():
+            out.zero_()
+            gemmainfer_csrc.fused_batched_moe(xd, Wd["gate_up_packed"], Wd["gate_up_scales"], Wd["down_packed"],
+                                              Wd["down_scales"], idxd, wd, out, gs)
+
+        call()
+        torch.cuda.synchronize()
+        first = out.clone()
+        assert_dtype_close(out, _oracle(W, x, idx, w, torch.zeros(m, h, dtype=dt), gs, tag), tag,
+                           f"few rows {tag} m={m}")
+        call()
+        torch.cuda.synchronize()
+        assert torch.equal(out, first)
+
+
 @pytest.mark.parametrize("tag", ["fp16", "fp32"])
 def test_moe_duplicates_invalid_ids_and_many_rows(tag):
     dt = DT[tag]
