@@ -257,9 +257,8 @@ def test_moe_fp16_grouped_gemm(h, i, e, k, gs, m):
 def test_moe_grouped_gemm_few_rows(tag, m):
     """The smallest calls on the grouped GEMM: the last row count of the 8-row
     launches (11) and the first here, one row tile per pass below 64 rows and
-    three above, an expert's
-    passes (none to more than 15, with every pair on
-    one expert), skipped ids, and the same bits from a second call."""
+    three from there, no pass to more than 15 of an expert (every pair on one),
+    skipped ids, and the same bits from a second call."""
     dt = torch.bfloat16 if tag == "bf16" else torch.float16
     h, i, e, k, gs = 256, 160, 40, 4, 64
     W = _moe_weights(e, h, i, gs, seed=970, dt=dt)
