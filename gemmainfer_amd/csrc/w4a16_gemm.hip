@@ -398,8 +398,9 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_small_kernel(GsArgs a) {
   const int colr = min(c0 + (GATED ? 4 * (lr & 7) : 4 * lr), sg.N - 4);
   const int32_t* bp = sg.B + colr;
   const uint16_t* sp = sg.S + colr;
-  int G = sg.G;
+  int G = sg.G, Gmax = sg.G;  // groups of the lane's columns; of the tile's
   if constexpr (GATED) {
+    Gmax = max(G, a.seg[1].G);
     if (lr >= 8) {
       bp = a.seg[1].B + colr;
       sp = a.seg[1].S + colr;
@@ -415,8 +416,12 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_small_kernel(GsArgs a) {
   for (int rt = 0; rt < RT; ++rt) roff[rt] = (uint32_t)min(rb * kRows + 16 * rt + lr, a.M - 1) * (uint32_t)a.K * 2u;
 
   // a unit past the wave's range, and a group past the scales, adds nothing:
-  // its token rows read zeros and its scales count as zero
-  const int kend = min(min(a.K, 32 * KPG * u1), G * a.gs);
+  // its token rows read zeros and its scales count as zero.  The token rows
+  // serve every lane's columns, so they end where the longer of two unequal
+  // scale tables does; the shorter one's columns end by their scales (there a
+  // non-finite value of the row is in the other factor of the result anyway).
+  const int kend = min(min(a.K, 32 * KPG * u1), Gmax * a.gs);
+  const int cend = min(kend, G * a.gs);
   u32x4_t xr[kAhead][RT][KPG], wr[kAhead][KPG];
   u32x2_t sr[kAhead];
   auto load = [&](int p, int u) {
@@ -458,7 +463,7 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_small_kernel(GsArgs a) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) B[s][q] = opaque(B[s][q]);  // unpacked here: the words' registers are free again
       }
-      const bool live = 32 * KPG * u < kend;
+      const bool live = 32 * KPG * u < cend;
       float sc[4] = {live ? moe::sc_lo<F16>(sr[p].x) : 0.f, live ? moe::sc_hi<F16>(sr[p].x) : 0.f,
                      live ? moe::sc_lo<F16>(sr[p].y) : 0.f, live ? moe::sc_hi<F16>(sr[p].y) : 0.f};
 #pragma unroll

@@ -59,6 +59,19 @@ def test_gemm_softcap_and_floor_groups(m):
     _check(y, 3.0 * np.tanh(ref / 3.0), torch.bfloat16)
 
 
+def _check_gated(got, g, u):
+    """gelu(g) * u of the projections' bf16 outputs, as the torch statements round it."""
+    want = torch.nn.functional.gelu(g.float(), approximate="tanh").to(torch.bfloat16) * u
+    # the two may sum K in different orders, so the rounding of a gate or up
+    # value may fall the other way: an ulp (at most 2^-7 of the value) of the
+    # gate through gelu's largest slope 1.13, of gelu's own rounding, of the up
+    # value, and of the result
+    g, u, w = g.float(), u.float(), want.float()
+    gel = torch.nn.functional.gelu(g, approximate="tanh")
+    bound = 2.0 ** -7 * ((1.13 * g.abs() + 2 * gel.abs()) * u.abs() + w.abs()) + 1e-6
+    assert torch.all((got.float() - w).abs() <= bound)
+
+
 @pytest.mark.parametrize("m", [24, 50, 1500])
 def test_gemm_multi_and_gated(m):
     """Several projections in one grid against the oracle; the gated form keeps the torch statements' roundings."""
@@ -69,16 +82,29 @@ def test_gemm_multi_and_gated(m):
         _check(y, O.w4a16_linear(_f64(x), B.cpu().numpy(), _f64(S), gs), torch.bfloat16)
     gate, up = (tuple(t.to(DEV) for t in synth.linear_weights(k, 1092, gs, seed=s)) for s in (7, 8))
     g, u = (ops.w4a16_linear(x, *w, gs) for w in (gate, up))
-    want = torch.nn.functional.gelu(g.float(), approximate="tanh").to(torch.bfloat16) * u
-    got = ops.gated_mlp_act(x, gate, up, gs)
-    # the two may sum K in different orders, so the rounding of a gate or up
-    # value may fall the other way: an ulp (at most 2^-7 of the value) of the
-    # gate through gelu's largest slope 1.13, of gelu's own rounding, of the up
-    # value, and of the result
-    g, u, w = g.float(), u.float(), want.float()
-    gel = torch.nn.functional.gelu(g, approximate="tanh")
-    bound = 2.0 ** -7 * ((1.13 * g.abs() + 2 * gel.abs()) * u.abs() + w.abs()) + 1e-6
-    assert torch.all((got.float() - w).abs() <= bound)
+    _check_gated(ops.gated_mlp_act(x, gate, up, gs), g, u)
+
+
+@pytest.mark.parametrize("gs", [64, 32])
+@pytest.mark.parametrize("m", [24, 50, 1500])
+def test_gated_unequal_group_counts(m, gs):
+    """Gate and up scales with different group counts (one covers all of K, the
+    other drops the rows of the last, partial group): every token row keeps
+    each projection's own rows, on the small tiles and on the large ones."""
+    k, n = 456, 1092
+    x = synth.activations(m, k, seed=m + gs).to(DEV)
+    gate, up = (tuple(t.to(DEV) for t in synth.linear_weights(k, n, gs, seed=s)) for s in (17, 18))
+
+    def short(w):
+        return w[0], w[1][: k // gs].contiguous()
+
+    def oracle(w):
+        kk = min(k, w[1].shape[0] * gs)
+        y = O.w4a16_linear(_f64(x)[:, :kk], w[0][: kk // 8].cpu().numpy(), _f64(w[1]), gs)
+        return torch.from_numpy(y).to(torch.bfloat16)
+
+    for gt, u in ((short(gate), up), (gate, short(up)), (short(gate), short(up))):
+        _check_gated(ops.gated_mlp_act(x, gt, u, gs).cpu(), oracle(gt), oracle(u))
 
 
 def test_gemm_output_at_any_element():
