@@ -145,10 +145,15 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GmArgs a) {
   const int colr = min(col, sg.N - 4);
   const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(sg.B, (uint32_t)((size_t)(a.K >> 3) * sg.N * 4));
   const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(sg.S, (uint32_t)((size_t)sg.G * sg.N * 2));
+  // k past the last scale group (the longer table's of GATED) is dropped: the
+  // fragments and offsets end there and read zeros beyond, since a zero scale
+  // alone would make NaN of an infinity or NaN in a dropped column
+  const int units = a.KBp / KPG, upg = a.gs / (32 * KPG);  // units of k; units per scale group
+  const int live = min(units, (GATED ? max(a.seg[0].G, a.seg[1].G) : sg.G) * upg);
   const __amdgpu_buffer_rsrc_t rx =
-      buffer_rsrc(a.xf + (size_t)(rb * kGmRT + wave) * a.KBp * kWave, (uint32_t)a.KBp * kWave * 16u);
+      buffer_rsrc(a.xf + (size_t)(rb * kGmRT + wave) * a.KBp * kWave, (uint32_t)(live * KPG) * kWave * 16u);
   const __amdgpu_buffer_rsrc_t ro =
-      buffer_rsrc(a.off + rb * kGmRows, F16 ? 0u : (uint32_t)((a.KBp / KPG - 1) * a.Mp + kGmRows) * 4u);
+      buffer_rsrc(a.off + rb * kGmRows, F16 ? 0u : (uint32_t)((live - 1) * a.Mp + kGmRows) * 4u);
   const uint32_t wstep = (uint32_t)sg.N * 16u;
   const uint32_t wbase = ((uint32_t)lq * (uint32_t)sg.N + (uint32_t)colr) * 4u;
   auto wload = [&](int kb) {
@@ -156,9 +161,8 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GmArgs a) {
     return make_uint4(v.x, v.y, v.z, v.w);
   };
   const uint32_t sbase = (uint32_t)colr * 2u, sstep = (uint32_t)sg.N * 2u;
-  const int upg = a.gs / (32 * KPG);  // units per scale group
   auto sload = [&](int u) {
-    // groups past the scales tensor read zeros (their rows are dropped)
+    // groups past the scales tensor read zeros
     const int g = u / upg;
     const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(rs, g < sg.G ? sbase + (uint32_t)g * sstep : 0xFFFFFFF0u, 0, 0);
     return make_uint2(v.x, v.y);
@@ -698,12 +702,17 @@ size_t gemm_workspace_bytes(int M, int K, int gs, const int* N, int n, bool gate
   return gm_plan(M, K, gs, N, n, gated).bytes;
 }
 
-// segs: the projections (gated: gate then up, the same N, out in segs[0].C);
+// given: the projections (gated: gate then up, the same N, out in given[0].C);
 // the caller checked gemm_supported, the tensors and the workspace's size.
-int launch_gemm(const void* A, bool f16, int M, int K, int gs, float cap, const GemmSeg* segs, int nseg, bool gated,
+int launch_gemm(const void* A, bool f16, int M, int K, int gs, float cap, const GemmSeg* given, int nseg, bool gated,
                 void* workspace, hipStream_t stream) {
   int N[kMaxGemmSegs];
-  for (int i = 0; i < nseg; ++i) N[i] = segs[i].N;
+  GemmSeg segs[kMaxGemmSegs];
+  for (int i = 0; i < nseg; ++i) {
+    segs[i] = given[i];
+    segs[i].G = min(given[i].G, (K + gs - 1) / gs);  // groups past K are never read: 32-bit sizes and offsets hold
+    N[i] = segs[i].N;
+  }
   const GmPlan p = gm_plan(M, K, gs, N, nseg, gated);
   if (p.small) return launch_small(A, f16, M, K, gs, cap, segs, nseg, gated, p, workspace, stream);
   const GmLayout l = gm_layout(M, K, gs);

@@ -46,17 +46,41 @@ def test_gemm_parity(m, k, n, gs, dtype):
     assert torch.equal(y, ops.w4a16_linear(x, B, S, gs))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m", [33, 1100])
-def test_gemm_softcap_and_floor_groups(m):
+def test_gemm_softcap_and_floor_groups(m, dtype):
     """Softcap epilogue; scales with fewer groups than K spans (the rows past
-    the last group are dropped)."""
+    the last group are dropped, an infinity or NaN in a dropped column with
+    them), on the small tiles and on the large ones; scales with more groups."""
     k, n, gs = 320, 2560, 128
-    x, B, S = _operands(m, k, n, gs, torch.bfloat16, seed=3)
+    x, B, S = _operands(m, k, n, gs, dtype, seed=3)
+    full = ops.w4a16_linear(x, B, S, gs, softcap=3.0)
+    assert torch.equal(full, ops.w4a16_linear(x, B, torch.cat([S, S + 1]), gs, softcap=3.0))
     S = S[: k // gs].contiguous()
+    x[3, 256], x[m - 1, 319], x[m // 2, 300] = float("inf"), float("nan"), float("-inf")
     y = ops.w4a16_linear(x, B, S, gs, softcap=3.0)
     kk = (k // gs) * gs
     ref = O.w4a16_linear(_f64(x)[:, :kk], B[: kk // 8].cpu().numpy(), _f64(S), gs)
-    _check(y, 3.0 * np.tanh(ref / 3.0), torch.bfloat16)
+    _check(y, 3.0 * np.tanh(ref / 3.0), dtype)
+
+
+@pytest.mark.parametrize("m", [40, 1100])
+def test_gemm_multi_unequal_group_counts(m):
+    """Projections of one call whose scales end at different groups: each drops
+    its own columns, with an infinity in one that only the first keeps."""
+    k, gs = 456, 64
+    x = synth.activations(m, k, seed=m).to(DEV)
+    x[5, 450] = float("inf")
+    ws = [tuple(t.to(DEV) for t in synth.linear_weights(k, n, gs, seed=n)) for n in (1092, 256, 520)]
+    ws[1] = (ws[1][0], ws[1][1][:7].contiguous())
+    ws[2] = (ws[2][0], ws[2][1][:4].contiguous())
+    ys = ops.w4a16_linear_multi(x, ws, gs)
+    keep = [i for i in range(m) if i != 5]
+    for i, (y, (B, S)) in enumerate(zip(ys, ws)):
+        kk = min(k, S.shape[0] * gs)
+        xi, yi = (x[keep], y[keep]) if i == 0 else (x, y)
+        _check(yi, O.w4a16_linear(_f64(xi)[:, :kk], B[: kk // 8].cpu().numpy(), _f64(S), gs), torch.bfloat16)
+    assert not torch.isfinite(ys[0][5].float()).any()
 
 
 def _check_gated(got, g, u):
