@@ -128,6 +128,7 @@ struct GemmSeg {
 };
 bool gemm_supported(int M, int K, int gs, const int* N, int n);
 size_t gemm_workspace_bytes(int M, int K, int gs, const int* N, int n, bool gated);
+size_t gemm_workspace_bound(int M, int K, int gs, const int* N, int n, bool gated);
 int launch_gemm(const void* A, bool f16, int M, int K, int gs, float cap, const GemmSeg* segs, int nseg, bool gated,
                 void* workspace, hipStream_t stream);
 

@@ -702,6 +702,25 @@ size_t gemm_workspace_bytes(int M, int K, int gs, const int* N, int n, bool gate
   return gm_plan(M, K, gs, N, n, gated).bytes;
 }
 
+// An upper bound of gemm_workspace_bytes over every row count up to M that
+// does not shrink as M grows (a plan's own need does: more rows need fewer K
+// slices, and the large kernel needs other buffers).  The small kernel splits
+// K only below kGsTargetWgs tiles, into ks <= kGsMaxSlices slices of ks * tiles
+// < kGsTargetWgs + tiles tiles; the large kernel's buffers grow with M.
+size_t gemm_workspace_bound(int M, int K, int gs, const int* N, int n, bool gated) {
+  const GmPlan p = gm_plan(M, K, gs, N, n, gated);
+  const size_t rows = M <= 32 ? 32 : 64;
+  size_t b = p.small ? 0 : p.bytes;
+  if (gm_tiles(N, n, gated, 64) < kGsTargetWgs) {
+    size_t tiles = p.tiles < kGsTargetWgs ? p.tiles : kGsTargetWgs - 1;
+    size_t slots = tiles + kGsTargetWgs - 1;
+    if (slots > tiles * kGsMaxSlices) slots = tiles * kGsMaxSlices;
+    const size_t s = gm_round(kGemmWsOffset + slots * rows * 64 * sizeof(float));
+    if (s > b) b = s;
+  }
+  return b;
+}
+
 // given: the projections (gated: gate then up, the same N, out in given[0].C);
 // the caller checked gemm_supported, the tensors and the workspace's size.
 int launch_gemm(const void* A, bool f16, int M, int K, int gs, float cap, const GemmSeg* given, int nseg, bool gated,

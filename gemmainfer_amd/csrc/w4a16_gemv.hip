@@ -1248,15 +1248,34 @@ Plan make_plan(int M, int K, int N) {
 
 }  // namespace
 
-size_t w4a16_workspace_bytes(int M, int K, int N, int gs) {
-  if (M <= 0 || K <= 0 || N <= 0) return 0;
+// The workspace queries do not shrink as M grows, so a workspace sized for a
+// program's largest M serves every smaller one.  Each path's need grows with M
+// except where the path changes, after 2, 8 and 16 rows: a query is the largest
+// of the path's own need and of the ones at those row counts below M.
+template <class Need>
+static size_t largest_need(int M, Need need) {
+  size_t b = need(M);
+  for (int m : {2, 8, 16}) {
+    if (m >= M) break;
+    const size_t x = need(m);
+    if (x > b) b = x;
+  }
+  return b;
+}
+
+static size_t linear_need(int M, int K, int N, int gs) {
   if (narrow_path(M, K, N)) return 0;
   if (gs > 0 && mfma_narrow_path(M, K, N, gs))
     return mn_workspace_bytes(M, K, (N + kMnCols - 1) / kMnCols, gs, false);
   // the matrix-core path needs none (scales with the full ceil(K / gs) groups)
   if (gs > 0 && mfma_path(M, K, N, gs, (K + gs - 1) / gs)) return 0;
-  if (gemm_supported(M, K, gs, &N, 1)) return gemm_workspace_bytes(M, K, gs, &N, 1, false);
+  if (gemm_supported(M, K, gs, &N, 1)) return gemm_workspace_bound(M, K, gs, &N, 1, false);
   return make_plan(M, K, N).total;
+}
+
+size_t w4a16_workspace_bytes(int M, int K, int N, int gs) {
+  if (M <= 0 || K <= 0 || N <= 0) return 0;
+  return largest_need(M, [&](int m) { return linear_need(m, K, N, gs); });
 }
 
 // Whether a call of more than 16 rows takes the matrix-core GEMM: its shape
@@ -1472,26 +1491,39 @@ int launch_w4a16_multi(const void* A, int n, const int32_t* const* B, const void
   return GI_OK;
 }
 
-size_t w4a16_multi_workspace_bytes(int n, const int* N, int M, int K, int gs) {
-  if (n <= 0 || n > kMaxSegs || !N || M <= 0 || K <= 0) return 0;
+static size_t multi_need(int n, const int* N, int M, int K, int gs) {
   if (narrow_multi(M, K, N, n)) return 0;
   if (gs > 0 && mfma_multi(M, K, N, n, gs)) return mn_workspace_bytes(M, K, mn_tiles(N, n), gs, false);
-  if (gemm_supported(M, K, gs, N, n)) return gemm_workspace_bytes(M, K, gs, N, n, false);
+  if (gemm_supported(M, K, gs, N, n)) return gemm_workspace_bound(M, K, gs, N, n, false);
   size_t b = 0;
   for (int i = 0; i < n; ++i) {
-    const size_t x = w4a16_workspace_bytes(M, K, N[i], gs);
+    const size_t x = N[i] > 0 ? linear_need(M, K, N[i], gs) : 0;
     if (x > b) b = x;
   }
   return b;
 }
 
-size_t w4a16_gated_workspace_bytes(int M, int K, int N, int gs) {
-  if (M <= 0 || K <= 0 || N <= 0) return 0;
+size_t w4a16_multi_workspace_bytes(int n, const int* N, int M, int K, int gs) {
+  if (n <= 0 || n > kMaxSegs || !N || M <= 0 || K <= 0) return 0;
+  return largest_need(M, [&](int m) { return multi_need(n, N, m, K, gs); });
+}
+
+// two linears into buffers behind their workspace, and an elementwise launch
+static size_t gated_two_need(int M, int K, int N) {
+  return gated_tmp_off(M, K, N) + 2 * round_up((size_t)M * N * 2);
+}
+
+static size_t gated_need(int M, int K, int N, int gs) {
   if (gated_narrow(M, K, N)) return 0;
   if (gs > 0 && gated_mfma(M, K, N, gs)) return mn_workspace_bytes(M, K, (N + kMnCols - 1) / kMnCols, gs, true);
   const int n2[2] = {N, N};
-  if (gemm_supported(M, K, gs, n2, 2)) return gemm_workspace_bytes(M, K, gs, n2, 2, true);
-  return gated_tmp_off(M, K, N) + 2 * round_up((size_t)M * N * 2);
+  if (gemm_supported(M, K, gs, n2, 2)) return gemm_workspace_bound(M, K, gs, n2, 2, true);
+  return gated_two_need(M, K, N);
+}
+
+size_t w4a16_gated_workspace_bytes(int M, int K, int N, int gs) {
+  if (M <= 0 || K <= 0 || N <= 0) return 0;
+  return largest_need(M, [&](int m) { return gated_need(m, K, N, gs); });
 }
 
 int launch_w4a16_gated(const void* A, const int32_t* gB, const void* gS, int gG, const int32_t* uB, const void* uS,
@@ -1513,15 +1545,15 @@ int launch_w4a16_gated(const void* A, const int32_t* gB, const void* gS, int gG,
                             GemmSeg{uB, (const uint16_t*)uS, nullptr, N, uG, 0}};
     return launch_gemm(A, false, M, K, gs, 0.f, gsg, 2, true, workspace, stream);
   }
-  const size_t need = w4a16_gated_workspace_bytes(M, K, N, gs);
-  if (!workspace || workspace_bytes < need || ((uintptr_t)workspace) % kAlign)
+  const size_t tmp = gated_tmp_off(M, K, N);  // the linears' own workspace ends here
+  if (!workspace || workspace_bytes < gated_two_need(M, K, N) || ((uintptr_t)workspace) % kAlign)
     return fail(GI_ERR_WORKSPACE, "w4a16_gated_mlp: workspace missing, misaligned or smaller than "
                                   "gi_w4a16_gated_mlp_workspace_bytes()");
-  uint16_t* tg = (uint16_t*)((char*)workspace + gated_tmp_off(M, K, N));
+  uint16_t* tg = (uint16_t*)((char*)workspace + tmp);
   uint16_t* tu = (uint16_t*)((char*)tg + round_up((size_t)M * N * 2));
-  st = launch_w4a16(A, gB, gS, gG, tg, M, K, N, gs, 0.f, workspace, workspace_bytes, stream);
+  st = launch_w4a16(A, gB, gS, gG, tg, M, K, N, gs, 0.f, workspace, tmp, stream);
   if (st != GI_OK) return st;
-  st = launch_w4a16(A, uB, uS, uG, tu, M, K, N, gs, 0.f, workspace, workspace_bytes, stream);
+  st = launch_w4a16(A, uB, uS, uG, tu, M, K, N, gs, 0.f, workspace, tmp, stream);
   if (st != GI_OK) return st;
   const int64_t n = (int64_t)M * N;
   const int blocks = (int)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);

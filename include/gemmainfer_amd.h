@@ -246,7 +246,9 @@ int gi_workspace_status(void* workspace, size_t workspace_bytes,
  * lm_head epilogue, gemma.py:356-357).  A, scales, C of a_dtype: bf16, fp16
  * or fp32 (marlin.cu:764-842; fp16 and fp32 run a VALU kernel with fp32
  * arithmetic and one rounding of C).  C is overwritten.  Requirements:
- * K % 8 == 0, N % 4 == 0 (bf16), group_size % 8 == 0.                       */
+ * K % 8 == 0, N % 4 == 0 (bf16), group_size % 8 == 0.  The workspace queries
+ * of this and the next two entries do not shrink as M grows: a workspace sized
+ * for the largest M serves every smaller one of the same shape.             */
 size_t gi_w4a16_workspace_bytes(int M, int K, int N, int group_size);
 int gi_w4a16_linear(const void* A, int a_dtype,
                     const int32_t* B_packed, const void* scales, int n_groups,

@@ -63,6 +63,23 @@ def test_workspace_queries_are_host_only(lib):
     assert lib.gi_w4a16_workspace_bytes(4, 16384, 2816, 128) > 0         # long K: VALU split-K partials
 
 
+@pytest.mark.parametrize("k,n,gs", [(2816, 4096, 64), (2816, 2112, 64), (2816, 262144, 128), (8192, 512, 128),
+                                    (2112, 2816, 64), (64, 4, 64), (200, 36, 32), (16384, 64, 256), (1712, 80000, 32),
+                                    (264, 1028, 8), (7768, 20480, 96)])
+def test_linear_workspace_queries_do_not_shrink(lib, k, n, gs):
+    """A workspace sized for the largest row count serves every smaller one:
+    the three linear queries never decrease as M grows, over all the paths a
+    row count can take."""
+    ns = (ctypes.c_int * 3)(n, n // 8 * 4 + 4, 4)
+    queries = {"linear": lambda m: lib.gi_w4a16_workspace_bytes(m, k, n, gs),
+               "gated": lambda m: lib.gi_w4a16_gated_mlp_workspace_bytes(m, k, n, gs),
+               "multi": lambda m: lib.gi_w4a16_linear_multi_workspace_bytes(3, ns, m, k, gs)}
+    for name, q in queries.items():
+        sizes = [(m, q(m)) for m in [*range(1, 140), *range(140, 1400, 13), 1500, 2048, 4096, 20000]]
+        for (m0, a), (m1, b) in zip(sizes, sizes[1:]):
+            assert a <= b, f"{name}: {a} bytes at {m0} rows, {b} at {m1}"
+
+
 def _moe_call(lib, **over):
     a = dict(x=ctypes.c_void_p(16), xd=L.DTYPE_BF16, gu=ctypes.c_void_p(16), gus=ctypes.c_void_p(16), ggu=22,
              dp=ctypes.c_void_p(16), ds=ctypes.c_void_p(16), gd=6, idx=ctypes.c_void_p(16), idt=L.DTYPE_INT32,

@@ -169,3 +169,31 @@ def test_gemm_without_its_workspace():
     assert st == L.GI_OK
     ref = O.w4a16_linear(_f64(x), B[:, :512].cpu().numpy(), _f64(S[:, :512]), gs)
     _check(y[:, :512], ref, torch.bfloat16)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("most", [320, 512, 1024])
+def test_one_workspace_for_the_largest_call(dtype, most):
+    """One workspace, sized for a program's largest row count, serves calls of
+    every smaller one, linear and gated, whatever their K
+    split: the same results as with a workspace of their own."""
+    k, n, gs = 2816, 4096, 64
+    lib, stream = L.load(), torch.cuda.current_stream().cuda_stream
+    p = lambda t: t.data_ptr()  # noqa: E731
+    code = L.DTYPE_BF16 if dtype == torch.bfloat16 else L.DTYPE_FP16
+    ws = torch.zeros(max(lib.gi_w4a16_workspace_bytes(most, k, n, gs),
+                         lib.gi_w4a16_gated_mlp_workspace_bytes(most, k, n, gs)) + 256, dtype=torch.uint8, device=DEV)
+    base = p(ws) + -p(ws) % 256
+    for m in (64, 17, 3, 192, 16, 64):
+        x, B, S = _operands(m, k, n, gs, dtype, seed=m)
+        y = torch.empty(m, n, dtype=dtype, device=DEV)
+        size = lib.gi_w4a16_workspace_bytes(most, k, n, gs)
+        assert lib.gi_w4a16_linear(p(x), code, p(B), p(S), S.shape[0], p(y), m, k, n, gs, 0.0, base, size,
+                                   stream) == L.GI_OK, (m, lib.gi_last_error())
+        assert torch.equal(y, ops.w4a16_linear(x, B, S, gs))
+        if dtype == torch.bfloat16:
+            size = lib.gi_w4a16_gated_mlp_workspace_bytes(most, k, n, gs)
+            S2 = S.flip(0).contiguous()
+            assert lib.gi_w4a16_gated_mlp(p(x), code, p(B), p(S), S.shape[0], p(B), p(S2), S.shape[0], p(y), m, k, n,
+                                          gs, base, size, stream) == L.GI_OK, (m, lib.gi_last_error())
+            assert torch.equal(y, ops.gated_mlp_act(x, (B, S), (B, S2), gs))
