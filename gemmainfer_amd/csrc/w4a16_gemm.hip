@@ -38,8 +38,8 @@ constexpr int kGmChunk = 4;      // k blocks (of 32) staged per barrier
 
 struct GmArgs {
   const uint4* xf;      // [row tiles][KBp][64] operand fragments
-  const float* off;     // [units][Mp]: -24 * sum of the row over the unit (bf16)
-  int M, K, KBp, Mp;    // KBp: k blocks padded to whole chunks; Mp: rows padded to whole blocks
+  const float* off;     // [row blocks][units][64 rows]: -24 * sum of the row over the unit (bf16)
+  int M, K, KBp;        // KBp: k blocks padded to whole chunks
   int gs, rb, total;    // rb row blocks; total workgroups
   int c8;               // every C is 8-byte aligned (a view may start at any element)
   float cap;
@@ -50,7 +50,7 @@ struct GmOrderArgs {
   const uint16_t* A;
   uint4* xf;
   float* off;
-  int M, K, KBp, Mp, units;
+  int M, K, KBp, units;
 };
 
 // One wave per (16-row tile, unit of KPG k blocks).
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256) void gemm_order_kernel(GmOrderArgs a) {
   if constexpr (!F16) {
     b += __shfl_xor(b, 16, kWave);
     b += __shfl_xor(b, 32, kWave);
-    if (lane < 16) a.off[(size_t)u * a.Mp + row] = b;
+    if (lane < 16) a.off[((size_t)(rt / kGmRT) * a.units + u) * kGmRows + row % kGmRows] = b;
   }
 }
 
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GmArgs a) {
   const __amdgpu_buffer_rsrc_t rx =
       buffer_rsrc(a.xf + (size_t)(rb * kGmRT + wave) * a.KBp * kWave, (uint32_t)(live * KPG) * kWave * 16u);
   const __amdgpu_buffer_rsrc_t ro =
-      buffer_rsrc(a.off + rb * kGmRows, F16 ? 0u : (uint32_t)((live - 1) * a.Mp + kGmRows) * 4u);
+      buffer_rsrc(a.off + (size_t)rb * units * kGmRows, F16 ? 0u : (uint32_t)(live * kGmRows) * 4u);
   const uint32_t wstep = (uint32_t)sg.N * 16u;
   const uint32_t wbase = ((uint32_t)lq * (uint32_t)sg.N + (uint32_t)colr) * 4u;
   auto wload = [&](int kb) {
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GmArgs a) {
     for (int j = 0; j < kGmChunk; ++j)
       ar[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, (uint32_t)((c * kGmChunk + j) * kWave + lane) * 16u, 0, 0);
     if constexpr (!F16)
-      orr = __builtin_amdgcn_raw_buffer_load_b32(ro, (uint32_t)((c * kUnits + wave) * a.Mp + lane) * 4u, 0, 0);
+      orr = __builtin_amdgcn_raw_buffer_load_b32(ro, (uint32_t)((c * kUnits + wave) * kGmRows + lane) * 4u, 0, 0);
   };
   auto astore = [&](int b) {
 #pragma unroll
@@ -585,7 +585,7 @@ GmLayout gm_layout(int M, int K, int gs) {
 
 template <int KPG, bool F16>
 int launch_gm(const GmOrderArgs& o, const GmArgs& k, bool gated, hipStream_t stream) {
-  hipLaunchKernelGGL((gemm_order_kernel<KPG, F16>), dim3((o.units + 3) / 4, o.Mp / 16), dim3(256), 0, stream, o);
+  hipLaunchKernelGGL((gemm_order_kernel<KPG, F16>), dim3((o.units + 3) / 4, k.rb * kGmRT), dim3(256), 0, stream, o);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "w4a16 gemm order launch");
   const dim3 grid(k.total), block(kGmThreads);
@@ -742,7 +742,6 @@ int launch_gemm(const void* A, bool f16, int M, int K, int gs, float cap, const 
   o.M = M;
   o.K = K;
   o.KBp = l.KBp;
-  o.Mp = l.Mp;
   o.units = l.units;
   GmArgs k{};
   k.xf = o.xf;
@@ -750,7 +749,6 @@ int launch_gemm(const void* A, bool f16, int M, int K, int gs, float cap, const 
   k.M = M;
   k.K = K;
   k.KBp = l.KBp;
-  k.Mp = l.Mp;
   k.gs = gs;
   k.rb = l.Mp / kGmRows;
   k.cap = cap;

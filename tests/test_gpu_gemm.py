@@ -197,3 +197,32 @@ def test_one_workspace_for_the_largest_call(dtype, most):
             assert lib.gi_w4a16_gated_mlp(p(x), code, p(B), p(S), S.shape[0], p(B), p(S2), S.shape[0], p(y), m, k, n,
                                           gs, base, size, stream) == L.GI_OK, (m, lib.gi_last_error())
             assert torch.equal(y, ops.gated_mlp_act(x, (B, S), (B, S2), gs))
+
+
+def test_gemm_rows_past_32_bit_offsets():
+    """2^19 + 400 rows of K 65536 at group size 32: the rows' offset table is
+    larger than 4 GiB (one offset per row and 32 k).  Rows from both ends and
+    around the 64-row blocks, the others zero."""
+    m, k, n, gs = 2 ** 19 + 400, 65536, 4, 32
+    if torch.cuda.mem_get_info()[0] < 180 * 2 ** 30:
+        pytest.skip("needs 180 GiB of free device memory")
+    _, B, S = _operands(1, k, n, gs, torch.bfloat16, seed=5)
+    rows = [0, 1, 63, 64, 2 ** 18 + 9, m - 81, m - 80, m - 6, m - 1]
+    xr = synth.activations(len(rows), k, seed=6)
+    lib = L.load()
+    size = lib.gi_w4a16_workspace_bytes(m, k, n, gs)
+    x = ws = None
+    try:
+        x = torch.zeros(m, k, dtype=torch.bfloat16, device=DEV)
+        x[torch.tensor(rows, device=DEV)] = xr.to(DEV)
+        ws, y = torch.zeros(size, dtype=torch.uint8, device=DEV), torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+        assert lib.gi_w4a16_linear(x.data_ptr(), L.DTYPE_BF16, B.data_ptr(), S.data_ptr(), S.shape[0], y.data_ptr(), m,
+                                   k, n, gs, 0.0, ws.data_ptr(), size,
+                                   torch.cuda.current_stream().cuda_stream) == L.GI_OK
+        y = y.cpu()
+    finally:
+        del x, ws
+        torch.cuda.empty_cache()
+    _check(y[rows], O.w4a16_linear(_f64(xr), B.cpu().numpy(), _f64(S), gs), torch.bfloat16)
+    y[rows] = 0
+    assert not y.any()
