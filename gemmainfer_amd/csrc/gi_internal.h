@@ -78,11 +78,11 @@ int launch_moe_decode1(const MoeHostArgs& h, void* state, int* status);
 // the same launches with the library's static per-GPU scratch (moe_static.hip)
 int launch_fused_moe_static(MoeHostArgs h);
 // prefill (moe_prefill.hip): sorted-by-expert grouped GEMM for M >= kPrefillMinRows
-// From 12 rows: launches of 8 rows read an expert's words again in each that
-// meets it.  Gemma shapes, group size 64, bf16, 8-row launches / grouped GEMM,
-// for tokens that choose their experts independently and for ones that agree
-// on most: 9 rows 78.9 / 69.2 and 55.2 / 60.4 us, 12 rows 100.9 / 72.4 and
-// 62.5 / 62.7 us, 16 rows 120.9 / 76.9 and 71.0 / 63.9 us.
+// The fewest rows of any shape there (pf_min_rows has the lines by shape):
+// launches of 8 rows read an expert's words again in each that meets it.  128
+// experts, top-8, Gemma widths, group size 64, bf16, 8-row launches / grouped
+// GEMM at 9 rows: 78.9 / 69.2 us for tokens that choose their experts
+// independently, 55.2 / 60.4 us for ones that agree on most.
 constexpr int kPrefillMinRows = 12;
 bool moe_prefill_supported(const MoeHostArgs& h);
 size_t moe_prefill_workspace_bytes(int M, int top_k, int H, int I, int E);

@@ -703,14 +703,44 @@ PfLayout pf_layout(int M, int top_k, int H, int I, int E) {
   return l;
 }
 
-// Row tiles per pass: one below 64 rows, where most experts have few pairs.
-// Above, tokens that agree on few experts fill three tiles: Gemma shapes,
-// group size 64, bf16, three / one at 64 rows 168.7 / 89.2 us for tokens that
-// choose independently, 118.7 / 143.8 us for ones that agree on most, 80 rows
-// 169.8 / 91.2 and 160.7 / 174.4 us.  (Several workgroups for an expert's
-// passes run those faster, 90 us at 80 rows, but the ones without a pass cost
-// the even case as much as it gains: 512 rows 199 / 282 us.)
-int pf_row_tiles(int M) { return M < 64 ? 1 : kPRT; }
+// Row tiles per pass.  Below 64 rows one, where most experts have few pairs;
+// three once the mean expert has more than 12 (then most have a second tile)
+// and a pass can hold more than 16, since a pass of three tiles costs about 1.4
+// of one tile's and a second pass 1.7.  Gemma widths, group size 64, bf16, one
+// / three: 8 experts, top-8, 17 rows 70.9 / 59.7 us, 40 rows 102.5 / 66.4; 16
+// experts, top-4, 49 rows 72.0 / 60.8 (tokens that choose independently) and
+// 128.4 / 108.5 (that agree on most); at a mean of 10, 40 rows of the latter
+// 44.2 / 59.8 and 101.1 / 64.2.  From 64 rows three: tokens that agree on few
+// experts fill them: 128 experts, top-8, three / one at 64 rows 168.7 / 89.2 us
+// (independent), 118.7 / 143.8 us (agreeing), 80 rows 169.8 / 91.2 and 160.7 /
+// 174.4 us.  (Several workgroups for an expert's passes run those faster, 90 us
+// at 80 rows, but the ones without a pass cost the even case as much as it
+// gains: 512 rows 199 / 282 us.)
+int pf_row_tiles(const MoeHostArgs& h) {
+  if (h.M >= 64) return kPRT;
+  return h.M > 16 && (long long)h.M * h.top_k > 12LL * h.E ? kPRT : 1;
+}
+
+// Rows from which this path is the faster one.  A launch of 8 rows reads at
+// most 8 top_k experts, so it is short where top_k is small or few experts
+// exist, while a pass here takes as long as H is wide.  At hidden sizes the
+// decode kernels serve (and above 2048, where a pass is longest), 8-row
+// launches / here, us, group size 64, bf16, tokens that choose their experts
+// independently and ones that agree on most:
+//   12 rows  E 128 top-8 100 / 71, 53 / 54;  E 32 top-8 68 / 46, 53 / 45;
+//            E 128 top-4 67 / 61, 43 / 51;   E 128 top-2 44 / 59, 42 / 49;
+//            E 8 top-2 37 / 41, 36 / 41;     E 8 top-8 40 / 43
+//   24 rows  E 128 top-8 171 / 79, 87 / 85;  E 32 top-8 120 / 48, 79 / 76;
+//            E 128 top-4 120 / 71, 75 / 80;  E 32 top-4 80 / 46, 60 / 72;
+//            E 8 top-2 56 / 42, 53 / 70;     E 8 top-8 59 / 72
+//   25 rows  E 128 top-2 89 / 62, 69 / 49;   E 8 top-2 70 / 42, 67 / 70;
+//            E 8 top-8 75 / 61
+// Narrower and wider shapes gain from 12 rows on (12 rows, E 8 top-2: H 1408
+// 34 / 31, H 512 27 / 19, H 4096 81 / 55).
+int pf_min_rows(const MoeHostArgs& h) {
+  const bool decode_widths = h.H > 2048 && h.H <= 2816 && h.I <= 768;
+  return decode_widths && (h.top_k < 6 || h.E < 2 * h.top_k) ? 25 : kPrefillMinRows;
+}
 
 template <int GSH, bool F16, int RT>
 int launch_products_gs(const MoeHostArgs& h, const PfArgs& k, const PfSlots& sl) {
@@ -751,7 +781,7 @@ int log2_exact(int v) {
 }  // namespace
 
 bool moe_prefill_supported(const MoeHostArgs& h) {
-  if (h.M < kPrefillMinRows) return false;
+  if (h.M < pf_min_rows(h)) return false;
   if (h.x_dtype != GI_DTYPE_BF16 && h.x_dtype != GI_DTYPE_FP16) return false;
   if (h.x_dtype == GI_DTYPE_FP16 && h.logits) return false;  // fp16 rows come with the caller's ids
   // fp16 rows, and fewer than 64 of bf16: operands that sit off 16 bytes, and
@@ -860,7 +890,7 @@ int launch_moe_prefill(const MoeHostArgs& h, void* workspace, size_t ws_bytes, i
   k.act_bytes = (uint32_t)((size_t)P * h.I * 2);
   const PfSlots sl{f.idx, w, f.idx_is64, w_dtype, h.E};
   const bool f16 = h.x_dtype == GI_DTYPE_FP16;
-  if (pf_row_tiles(h.M) == 1) return f16 ? launch_products<true, 1>(h, k, sl) : launch_products<false, 1>(h, k, sl);
+  if (pf_row_tiles(h) == 1) return f16 ? launch_products<true, 1>(h, k, sl) : launch_products<false, 1>(h, k, sl);
   return f16 ? launch_products<true, kPRT>(h, k, sl) : launch_products<false, kPRT>(h, k, sl);
 }
 

@@ -104,6 +104,18 @@ def assert_dtype_close(got: torch.Tensor, ref64: np.ndarray, dtype: str, what: s
     return stats
 
 
+def kernels_of(call) -> list:
+    """Names of the GPU kernels that ``call`` launches, in order."""
+    from torch.profiler import ProfilerActivity, profile
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        call()
+        torch.cuda.synchronize()
+    names = [e.name for e in p.events() if e.device_type == torch.autograd.DeviceType.CUDA]
+    assert names, "the profiler recorded no kernel"
+    return names
+
+
 # Error statistics of the BASELINE configs' parity tests, by config name;
 # tests/conftest.py writes them to the JSON file named by GI_PARITY_STATS
 # at the end of the session (when that variable is set).

@@ -10,7 +10,7 @@ import torch
 from gemmainfer_amd import ops, synth
 from gemmainfer_amd import _lib as L
 from oracle import moe_oracle as O
-from tests.helpers import assert_bf16_close, assert_logits_close, np64, record_parity
+from tests.helpers import assert_bf16_close, assert_dtype_close, assert_logits_close, kernels_of, np64, record_parity
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -289,6 +289,46 @@ def test_prefill_scale_table_at_lds_limit(I):
                           Wd["down_scales"], idx.to(DEV), w.to(DEV), out, gs)
     ref, _ = _oracle_moe(x, W, idx, w, torch.zeros(m, H), gs)
     assert_bf16_close(out, ref, f"prefill I={I} gs32")
+
+
+# (rows, experts, top_k, H): row tiles per pass of the grouped GEMM, 0 for
+# launches of 8 rows; the lines of the rule at a decode width and a narrow one
+MOE_ROUTES = [(11, 16, 8, 512, 0), (12, 16, 8, 2816, 1), (24, 16, 8, 2816, 1), (25, 16, 8, 2816, 3),
+              (24, 8, 8, 2816, 0), (25, 8, 8, 2816, 3), (24, 8, 2, 2816, 0), (25, 8, 2, 2816, 1), (12, 8, 2, 512, 1),
+              (48, 8, 2, 512, 1), (49, 8, 2, 512, 3), (16, 1, 1, 512, 1), (17, 1, 1, 512, 3), (63, 64, 2, 512, 1),
+              (64, 64, 2, 512, 3)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,e,top_k,h,tiles", MOE_ROUTES)
+def test_route_by_rows_and_experts(m, e, top_k, h, tiles, dtype):
+    """Which kernels a call of 11 to 64 rows takes, by rows, experts, top_k and
+    hidden size, and its result there."""
+    i, gs = 128, 64
+    W = synth.moe_weights(E=e, H=h, I=i, group_size=gs, seed=e + h)
+    for n in ("gate_up_scales", "down_scales"):
+        W[n] = W[n].to(dtype)
+    Wd = _dev(W)
+    g = torch.Generator().manual_seed(m)
+    idx = torch.stack([torch.randperm(e, generator=g)[:top_k] for _ in range(m)]).to(torch.int32)
+    w = (torch.rand(m, top_k, generator=g) / top_k).to(dtype)
+    x = synth.activations(m, h, seed=m).to(dtype)
+    xd, idxd, wd = x.to(DEV), idx.to(DEV), w.to(DEV)
+    out = torch.zeros(m, h, dtype=dtype, device=DEV)
+    call = lambda: ops.fused_batched_moe(xd, Wd["gate_up_packed"], Wd["gate_up_scales"], Wd["down_packed"],  # noqa: E731
+                                         Wd["down_scales"], idxd, wd, out, gs)
+    call()
+    tag = "bf16" if dtype == torch.bfloat16 else "fp16"
+    ref, _ = O.fused_batched_moe(np64(x), W["gate_up_packed"].numpy(), np64(W["gate_up_scales"]),
+                                 W["down_packed"].numpy(), np64(W["down_scales"]), idx.numpy(), np64(w),
+                                 np.zeros((m, h)), gs, dtype=tag)
+    assert_dtype_close(out, ref, tag, f"m={m} E={e} k={top_k} H={h}")
+    names = kernels_of(call)
+    gu = [n for n in names if "prefill_gu_kernel" in n]
+    if tiles:
+        assert len(names) == 4 and len(gu) == 1 and f", {tiles}>" in gu[0], names
+    else:
+        assert not gu and len(names) == (m + 7) // 8, names
 
 
 @pytest.mark.parametrize("m", [100, 512])
