@@ -622,7 +622,7 @@ GmPlan gm_plan(int M, int K, int gs, const int* N, int n, bool gated) {
   GmPlan p{};
   const int kpg = gm_kpg(gs), units = (K + 32 * kpg - 1) / (32 * kpg);
   const GmLayout l = gm_layout(M, K, gs);
-  p.rt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+  p.rt = M <= 32 ? 2 : 4;
   p.rb = (M + 16 * p.rt - 1) / (16 * p.rt);
   p.tiles = gm_tiles(N, n, gated, 64) * p.rb;
   const long large = (long)gm_tiles(N, n, gated, kGmCols) * (l.Mp / kGmRows);
@@ -651,7 +651,6 @@ int launch_gs(const GsArgs& k, int tiles, bool gated, hipStream_t stream) {
 }
 template <int KPG, bool F16>
 int launch_gs_rt(const GsArgs& k, const GmPlan& p, bool gated, hipStream_t stream) {
-  if (p.rt == 1) return launch_gs<KPG, 1, F16>(k, p.tiles, gated, stream);
   if (p.rt == 2) return launch_gs<KPG, 2, F16>(k, p.tiles, gated, stream);
   return launch_gs<KPG, 4, F16>(k, p.tiles, gated, stream);
 }
