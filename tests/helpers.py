@@ -105,14 +105,15 @@ def assert_dtype_close(got: torch.Tensor, ref64: np.ndarray, dtype: str, what: s
 
 
 def kernels_of(call) -> list:
-    """Names of the GPU kernels that ``call`` launches, in order."""
+    """Names of the library's kernels that ``call`` launches, in order (torch's
+    own, such as a workspace's zero fill, left out)."""
     from torch.profiler import ProfilerActivity, profile
     torch.cuda.synchronize()
     with profile(activities=[ProfilerActivity.CUDA]) as p:
         call()
         torch.cuda.synchronize()
-    names = [e.name for e in p.events() if e.device_type == torch.autograd.DeviceType.CUDA]
-    assert names, "the profiler recorded no kernel"
+    names = [e.name for e in p.events() if e.device_type == torch.autograd.DeviceType.CUDA and "gi::" in e.name]
+    assert names, "the profiler recorded no kernel of the library"
     return names
 
 

@@ -29,11 +29,13 @@ def _check(y, ref, dtype):
 
 
 # rows: one past 16, the 16-, 32- and 64-row tiles' edges, several row blocks;
-# columns: N = 4 mod 64 and mod 256, one tile; K: 8 mod 32, less than a unit, a
-# last group cut short, one past a chunk; enough tiles for the large kernel
-SHAPES = [(17, 64, 64, 64), (32, 136, 68, 64), (33, 512, 200, 64), (64, 2816, 260, 64), (65, 704, 132, 128),
-          (40, 96, 68, 32), (70, 200, 36, 64), (61, 1000, 300, 192), (16 * 5 + 1, 264, 4, 96), (129, 8200, 64, 64),
-          (1281, 264, 2052, 64), (1300, 520, 2304, 32), (2049, 200, 1284, 128), (640, 2816, 4096, 64)]
+# one and two k blocks per unit at each row tile count; columns: N = 4 mod 64 and
+# mod 256, one tile; K: 8 mod 32, less than a unit, a last group cut short, one
+# past a chunk; enough tiles for the large kernel
+SHAPES = [(17, 64, 64, 64), (17, 264, 132, 32), (32, 200, 68, 96), (32, 136, 68, 64), (33, 512, 200, 64),
+          (64, 2816, 260, 64), (65, 704, 132, 128), (40, 96, 68, 32), (70, 200, 36, 64), (61, 1000, 300, 192),
+          (16 * 5 + 1, 264, 4, 96), (129, 8200, 64, 64), (1281, 264, 2052, 64), (1300, 520, 2304, 32),
+          (2049, 200, 1284, 128), (640, 2816, 4096, 64)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -132,8 +134,8 @@ def test_gated_unequal_group_counts(m, gs):
 
 
 def test_gemm_output_at_any_element():
-    """An output that starts at an odd element (2-byte aligned only), and a
-    strided one, through the drop-in's write semantics."""
+    """An output that starts at an odd element (2-byte aligned only), and one
+    whose rows are strided, through the drop-in's write semantics."""
     for m in (30, 1200):
         k, n, gs = 264, 2564, 64
         x, B, S = _operands(m, k, n, gs, torch.bfloat16, seed=1)
@@ -142,6 +144,9 @@ def test_gemm_output_at_any_element():
         C = flat[3:].view(m, n)
         ops.marlin_w4a16(x, B, S, C, gs)
         assert torch.equal(C, want) and not flat[:3].any()
+        wide = torch.zeros(m, n + 5, dtype=torch.bfloat16, device=DEV)
+        ops.marlin_w4a16(x, B, S, wide[:, 3:n + 3], gs)
+        assert torch.equal(wide[:, 3:n + 3], want) and not wide[:, :3].any() and not wide[:, n + 3:].any()
 
 
 def test_gemm_rows_with_inf_stay_apart():

@@ -176,8 +176,9 @@ def test_fused_gemma_shapes_gs128(gemma128, m, noise):
 
 @pytest.mark.parametrize("m", [64, 512])
 def test_prefill_grouped_gemm_gemma(gemma128, m):
-    """From 64 rows the sorted-by-expert grouped GEMM replaces the 8-row slices
-    (gemma.py:99-112): BASELINE config 3 at m=512, i.i.d. router logits."""
+    """The sorted-by-expert grouped GEMM, with three row tiles per pass, in the
+    place of the 8-row slices (gemma.py:99-112): 64 rows, the fewest of that
+    form at these shapes, and a prefill of 512 with i.i.d. router logits."""
     W, Wd = gemma128
     x = synth.activations(m, 2816, seed=500 + m)
     logits = synth.router_logits(m, 128, seed=500 + m)
@@ -221,9 +222,8 @@ def test_prefill_duplicates_invalid_skewed(small):
                                                (96, 16, torch.int32)])
 def test_prefill_many_pairs_and_heavy_expert(small, m, top_k, idx_dtype):
     """The front launch's align sorts up to 8192 (token, slot) pairs from
-    registers (1024 x 8 is the largest such call, 64 x 1 the smallest prefill
-    call) and more in a loop (1025 x 8); top_k 16 takes the combine's general
-    form.  Eight experts take ~500-1000 pairs
+    registers (1024 x 8 is the largest such call, 64 x 1 a single wave's worth)
+    and more in a loop (1025 x 8); top_k 16 takes the combine's general form.  Eight experts take ~500-1000 pairs
     each, i.e. 11-22 passes of 48 pairs per workgroup, and one expert takes
     most of them; ids outside [0, E) are skipped, duplicate ids within a
     token each count, and the output is the same on a second call."""
@@ -331,6 +331,36 @@ def test_route_by_rows_and_experts(m, e, top_k, h, tiles, dtype):
         assert not gu and len(names) == (m + 7) // 8, names
 
 
+@pytest.mark.parametrize("h,i,gs", [(320, 160, 128), (256, 128, 64)])
+@pytest.mark.parametrize("m", [20, 45])
+def test_few_rows_off_the_grouped_gemm(m, h, i, gs):
+    """bf16 calls of 12 to 63 rows that the launches of 8 rows keep: out 8 bytes
+    past a multiple of 16, and scales that end before K (the rows they do not
+    cover are dropped); layer and drop-in, against the oracle."""
+    e, k = 16, 4
+    W = synth.moe_weights(E=e, H=h, I=i, group_size=gs, seed=h + m)
+    short = {**W, "gate_up_scales": W["gate_up_scales"][:, :-1].contiguous(),
+             "down_scales": W["down_scales"][:, :-1].contiguous()}
+    x = synth.activations(m, h, seed=m)
+    logits = synth.router_logits(m, e, seed=m)
+    for V, off in ((W, 4), (short, 0), (short, 4)):
+        Vd = _dev(V)
+        ws = (Vd["gate_up_packed"], Vd["gate_up_scales"], Vd["down_packed"], Vd["down_scales"])
+        out = torch.zeros(m * h + off, dtype=torch.bfloat16, device=DEV)[off:].view(m, h)
+        xd, logits_d, res = x.to(DEV), logits.to(DEV), []
+        names = kernels_of(lambda: res.append(ops.moe_layer(xd, logits_d, *ws, k, gs, out=out)))
+        assert len(names) == (m + 7) // 8 and not any("prefill" in n for n in names), names
+        _, idx, w = res[0]
+        ref, ref_idx, _, _ = O.moe_layer_from_logits(
+            np64(x), np64(logits), V["gate_up_packed"].numpy(), np64(V["gate_up_scales"]), V["down_packed"].numpy(),
+            np64(V["down_scales"]), k, gs)
+        np.testing.assert_array_equal(idx.cpu().numpy(), ref_idx)
+        assert_bf16_close(out, ref, f"layer m={m} off={off} groups={V['gate_up_scales'].shape[1]}")
+        out.zero_()
+        ops.fused_batched_moe(xd, *ws, idx, w, out, gs)
+        assert_bf16_close(out, ref, f"drop-in m={m} off={off} groups={V['gate_up_scales'].shape[1]}")
+
+
 @pytest.mark.parametrize("m", [100, 512])
 def test_prefill_layer_matches_oracle_and_is_deterministic(gemma128, m):
     """Layer mode through the prefill path: routing bit-exact, output within
@@ -355,14 +385,18 @@ def test_prefill_layer_matches_oracle_and_is_deterministic(gemma128, m):
 
 
 def test_layer_from_logits_gemma(gemma128):
-    """Layer mode; 12 and 16 rows take several launches of up to 8 rows each."""
+    """Layer mode: one launch (1 and 7 rows), several launches of up to 8 rows
+    (9 and 11), the grouped GEMM (12 and 16)."""
     W, Wd = gemma128
-    for m, noise in ((1, 0.0), (7, 0.5), (12, 0.5), (16, 0.0)):
+    for m, noise in ((1, 0.0), (7, 0.5), (9, 0.0), (11, 0.5), (12, 0.5), (16, 0.0)):
         x = synth.activations(m, 2816, seed=10 + m)
         logits = synth.router_logits(m, 128, seed=10 + m, verify_noise=noise)
-        out, idx, w = ops.moe_layer(x.to(DEV), logits.to(DEV), Wd["gate_up_packed"],
-                                    Wd["gate_up_scales"], Wd["down_packed"], Wd["down_scales"],
-                                    8, 128)
+        xd, logits_d, res = x.to(DEV), logits.to(DEV), []
+        names = kernels_of(lambda: res.append(ops.moe_layer(
+            xd, logits_d, Wd["gate_up_packed"], Wd["gate_up_scales"], Wd["down_packed"], Wd["down_scales"], 8, 128)))
+        out, idx, w = res[0]
+        grouped = any("prefill_gu_kernel" in n for n in names)
+        assert grouped if m >= 12 else not grouped and len(names) == (m + 7) // 8, (m, names)
         ref_out, ref_idx, ref_w, al = O.moe_layer_from_logits(
             np64(x), np64(logits), W["gate_up_packed"].numpy(), np64(W["gate_up_scales"]),
             W["down_packed"].numpy(), np64(W["down_scales"]), 8, 128)
