@@ -1,8 +1,10 @@
 // fp16 and fp32 activations for the two drop-in entry points: the reference
 // dispatches bf16, fp16 and fp32 (csrc/marlin.cu:694-700 for the MoE,
-// :764-770, :816-822, :831-842 for the linear).  bf16 runs the tuned kernels;
-// these VALU kernels serve the other two dtypes with fp32 arithmetic and the
-// reference's rounding points in the activation dtype T:
+// :764-770, :816-822, :831-842 for the linear).  bf16 runs the tuned kernels,
+// and fp16 does in linears of more than 16 rows and in the MoE calls that the
+// decode kernels or the grouped GEMM take; these VALU kernels serve fp32 and
+// the other fp16 calls with fp32 arithmetic and the reference's rounding points
+// in the activation dtype T:
 //   * the routing weights are cast to T (marlin.cu:634-636),
 //   * the activation gelu_tanh(gate) * up is stored in T (:421-423),
 //   * the output is rounded to T (the MoE adds to out: :583, one rounding

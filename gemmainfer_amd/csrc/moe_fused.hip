@@ -1174,10 +1174,11 @@ int launch_fused_moe(const MoeHostArgs& h) {
                               (int*)((char*)h.workspace + L.ctr) + 4 * kCtrStride);
   }
   if (h.x_dtype == GI_DTYPE_FP16) {
-    // fp16 rows that the grouped GEMM does not take.  One token: the one-token kernel's fp16 variant (split bf16
-    // operands); more rows: the 8-row kernel's fp16 variant (fp16 products on
-    // q - 8 operands), one launch per 8 rows (~30 us each at the Gemma shapes,
-    // against ~120 us for the VALU kernels' launch of 64 slots)
+    // fp16 rows that the grouped GEMM does not take.  One token: the one-token
+    // kernel's fp16 variant (split bf16 operands); more rows: the 8-row
+    // kernel's fp16 variant (fp16 products on q - 8 operands), one launch per 8
+    // rows (~30 us each at the Gemma shapes, against ~120 us for the VALU
+    // kernels' launch of 64 slots)
     const int per = moe_rows_per_launch(h.top_k);
     const WsLayout L = ws_layout((h.M < per ? h.M : per) * h.top_k, h.H, h.I, kTaskCols);
     char* ws0 = (char*)h.workspace;

@@ -363,8 +363,8 @@ __device__ __forceinline__ void grouped_products(__amdgpu_buffer_rsrc_t rw, uint
         if constexpr (!F16) Db[rt] = moe::mfma_bf16(A, bc, gstart ? zf : Db[rt]);
       }
       // issue order: the A reads, then each product followed by three VALU
-      // operations (the next word's unpack; four in fp16, which subtracts 152), so that one wave's unpack runs
-      // under its own products (left to itself the compiler puts the whole
+      // operations (the next word's unpack; four in fp16, which subtracts 152),
+      // so that one wave's unpack runs under its own products (left to itself the compiler puts the whole
       // unpack first: gate/up 111-113 -> 108 us at M=512)
       __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);  // LDS reads
 #pragma unroll
@@ -435,8 +435,8 @@ __device__ __forceinline__ ScaleStage<ColOf> scale_stage(const uint16_t* sc_e, i
 // with the row tile's sums in the chunk buffers (free by then), a third of the
 // buffers and 168 registers three workgroups fit a CU instead of two: more of
 // the words are in flight, which is what bounds a small batch.  29 rows that
-// choose independently (Gemma shapes, group size 64, bf16): 220.9 us as 8-row
-// launches, 82.4 us here.
+// choose independently (Gemma shapes, 128 experts, top-8, group size 64, bf16):
+// 220.9 us as 8-row launches, 82.4 us here.
 template <int GSH, bool F16, int RT>
 __global__ __launch_bounds__(kPThreads, RT == 1 ? 3 : 2) void prefill_gu_kernel(PfArgs a) {
   __shared__ uint4 aring[2 * kPChunk * RT * 64 + (RT == 1 ? 0 : 1024)];
@@ -552,8 +552,8 @@ __global__ __launch_bounds__(kPThreads, RT == 1 ? 3 : 2) void prefill_down_kerne
 // ---------------------------------------------------------------------------
 // A pair's routing as the combine reads it: whether its id is in [0, E)
 // (other ids are skipped, marlin.cu:288-289) and its weight rounded to the
-// activation dtype (marlin.cu:631-636), from the caller's (or the routed) ids and weights.
-// Its result row is the pair index itself.
+// activation dtype (marlin.cu:631-636), from the caller's (or the routed) ids
+// and weights.  Its result row is the pair index itself.
 struct PfSlots {
   const void* idx;
   const void* w;

@@ -162,7 +162,8 @@ _ACT_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 
 def _require_act_dtype(x: torch.Tensor, who: str) -> None:
     """bf16, fp16 or fp32 activations (the reference's dispatch, marlin.cu:694-700,
-    :764-842): bf16 runs the tuned kernels, fp16 and fp32 VALU kernels."""
+    :764-842).  bf16 runs the tuned kernels; so do fp16 MoE calls (caller-given
+    ids) and fp16 linears of more than 16 rows; the rest run VALU kernels."""
     if x.dtype not in _ACT_DTYPES:
         raise TypeError(f"{who}: activations must be bf16, fp16 or fp32; got {x.dtype}")
 
@@ -222,8 +223,9 @@ def fused_batched_moe(x, gate_up_packed, gate_up_scales, down_packed, down_scale
 def moe_layer(x, router_logits, gate_up_packed, gate_up_scales, down_packed, down_scales,
               top_k, group_size, expert_scale=None, out=None, *, spin_limit: int = 0):
     """Router tail + fused MoE (gemma.py:77-98): one launch per 8 rows up to
-    11 rows, and from 12 rows the grouped-GEMM prefill path (routing, align,
-    gate/up, down and combine launches).
+    11 rows (up to 24 at decode widths with few experts or a small top_k), and
+    from there the grouped-GEMM prefill path (routing with the align, gate/up,
+    down and combine launches).
 
     Returns (out [M, H] bf16 -- overwritten, idx int32 [M, top_k],
     weights bf16 [M, top_k]).
@@ -438,7 +440,8 @@ def _linear_operands(A, B_packed, scales, who):
 
 def w4a16_linear_multi(A, weights, group_size):
     """Several W4A16 projections of the same rows (the q, k, v marlin_w4a16 calls
-    of attention.py:115-122) in one call: one launch for one or two rows.
+    of attention.py:115-122) in one grid: one launch, two (the rows' order and
+    the products) where the call has enough rows to fill the chip.
     ``weights`` is a list of up to 4 (B_packed, scales); returns the outputs."""
     dev = _on_device(A, *[t for w in weights for t in w])
     _require_bf16(A, "w4a16_linear_multi")
@@ -466,8 +469,8 @@ def w4a16_linear_multi(A, weights, group_size):
 
 def gated_mlp_act(A, gate, up, group_size):
     """GemmaMLP's ``gelu_tanh(gate_proj(x)) * up_proj(x)`` (activations.py:26-28)
-    with the bf16 roundings of those torch statements; one launch for one or
-    two rows.  ``gate`` and ``up`` are (B_packed, scales); returns bf16 [M, N]."""
+    with the bf16 roundings of those torch statements, in one grid as in
+    ``w4a16_linear_multi``.  ``gate`` and ``up`` are (B_packed, scales); returns bf16 [M, N]."""
     dev = _on_device(A, *gate, *up)
     _require_bf16(A, "gated_mlp_act")
     _require(A.dim() == 2, "A must be [M, K]")

@@ -114,16 +114,19 @@ int gi_moe_align(const void* idx, int idx_dtype, int M, int top_k, int E,
  *   idx        int32|int64 [M*top_k]  w  bf16|fp16|fp32 [M*top_k]
  *   out        T [M, H]               accumulated into (caller zeroes it)
  * T = x_dtype: bf16, fp16 or fp32 (marlin.cu:694-700).  bf16 runs the paths
- * below, and so does fp16 where operands are 16-byte aligned and the scales
- * cover K; other fp16 and fp32 calls run VALU kernels (fp32 arithmetic, the routing
+ * below, and so does fp16 at the decode kernel's shapes and on the prefill
+ * path; other fp16 and fp32 calls run VALU kernels (fp32 arithmetic, the routing
  * weights cast to T, the activation stored in T, one rounding of the output
  * in T; the dequantised weights are never rounded; Token-Union in launches
  * of up to 64 slots, top_k <= 64: alignment, gate/up, down, combine).
- * One kernel launch per 256/top_k rows (8 rows on the decode kernel); from
- * 12 rows with top_k <= 64, a power-of-two multiple of 32 as group size,
- * H % 64 == 0 and I % 32 == 0, the grouped-GEMM prefill path (align with
- * the x reorder, gate/up, down, combine launches; each active expert read
- * once).
+ * One kernel launch per 256/top_k rows (8 rows on the decode kernel and for
+ * group sizes that are multiples of 32).  From 12 rows (25 where 2048 < H <=
+ * 2816, I <= 768 and top_k < 6 or E < 2 * top_k) with top_k <= 64, a
+ * power-of-two multiple of 32 up to 256 as group size, H % 64 == 0 and
+ * I % 32 == 0, the grouped-GEMM prefill path (align with the x reorder,
+ * gate/up, down, combine launches; each active expert read once); fp16 calls,
+ * and bf16 ones below 64 rows, take it where x, weights, scales and out are
+ * 16-byte aligned and the scales cover H and I.
  * Requirements: H % 8 == 0,
  * I % 8 == 0, H, I multiples of 4 columns, group_size % 8 == 0, E <= 1024,
  * top_k <= 256.  Deterministic (fixed-order fp32 reductions, no float
@@ -180,8 +183,8 @@ int gi_fused_batched_moe_static_status(int32_t* host_status, int clear, void* st
 /* Router + fused MoE: logits [M, E] (bf16/fp32) are routed as
  * gi_moe_route_topk_softmax does (weights rounded to bf16), out[M, H] is
  * OVERWRITTEN with the MoE output, and out_idx/out_w (may be NULL) receive
- * the routing.  Up to 8 rows per launch; from 12 rows (group size a power of
- * two times 32, H % 64 == 0, I % 32 == 0) the sorted-by-expert grouped-GEMM
+ * the routing.  Up to 8 rows per launch; from 12 rows (or 25, under the same
+ * conditions as gi_fused_batched_moe) the sorted-by-expert grouped-GEMM
  * prefill path replaces the 8-row slices of gemma.py:99-112 (routing with
  * the align and the x reorder, gate/up, down, combine launches).           */
 int gi_moe_layer_from_logits(const void* x, int x_dtype,
@@ -244,9 +247,13 @@ int gi_workspace_status(void* workspace, size_t workspace_bytes,
  * C[M, N] = A[M, K] @ dequant(B_packed[K/8, N], scales[n_groups, N]),
  * optionally followed by C = softcap*tanh(C/softcap) when softcap > 0 (the
  * lm_head epilogue, gemma.py:356-357).  A, scales, C of a_dtype: bf16, fp16
- * or fp32 (marlin.cu:764-842; fp16 and fp32 run a VALU kernel with fp32
- * arithmetic and one rounding of C).  C is overwritten.  Requirements:
- * K % 8 == 0, N % 4 == 0 (bf16), group_size % 8 == 0.  The workspace queries
+ * or fp32 (marlin.cu:764-842), one rounding of C.  bf16 and fp16 calls of more
+ * than 16 rows run a matrix-core GEMM (group_size % 32 == 0, N % 4 == 0, A and
+ * B_packed 16-byte and scales 8-byte aligned; a workspace smaller than the
+ * query, or an unmet condition, sends fp16 to the VALU kernel, and bf16 to one
+ * where the workspace holds its partials); fp32 and other fp16 calls run a
+ * VALU kernel with fp32 arithmetic.  C is overwritten.  Requirements: K % 8
+ * == 0, N % 4 == 0 (bf16), group_size % 8 == 0.  The workspace queries
  * of this and the next two entries do not shrink as M grows: a workspace sized
  * for the largest M serves every smaller one of the same shape.             */
 size_t gi_w4a16_workspace_bytes(int M, int K, int N, int group_size);
@@ -261,7 +268,9 @@ int gi_w4a16_linear(const void* A, int a_dtype,
  * input there).  C[i][M, N[i]] = A @ dequant(B_packed[i], scales[i]) for
  * i < n_proj <= 4.  One launch for 1-2 rows (16-column tiles of every
  * projection in one grid) and for 3-16 rows on the matrix-core path (64-column
- * tiles); otherwise one gi_w4a16_linear per projection, in order.  Size the
+ * tiles); the GEMM's one or two launches, all projections in one grid, past 16
+ * rows (group_size % 32 == 0); otherwise one gi_w4a16_linear per projection, in
+ * order.  Size the
  * workspace with gi_w4a16_linear_multi_workspace_bytes.  Arrays are host
  * memory.                                                                    */
 size_t gi_w4a16_linear_multi_workspace_bytes(int n_proj, const int* N, int M, int K,
@@ -276,9 +285,11 @@ int gi_w4a16_linear_multi(const void* A, int a_dtype, int n_proj,
  *   out[M, N] = bf16( bf16(gelu_tanh(bf16(A @ Wg))) * bf16(A @ Wu) )
  * with the bf16 roundings of the torch statements.  One launch for 1-2 rows
  * (16-column tiles) and for 3-16 rows on the matrix-core path (both
- * projections per 64-column tile, the gelu and product in the epilogue).
- * Otherwise two linears into the workspace and an elementwise launch; size
- * the workspace with gi_w4a16_gated_mlp_workspace_bytes.                   */
+ * projections per 64-column tile, the gelu and product in the epilogue); the
+ * GEMM's one or two launches with the same epilogue past 16 rows (group_size %
+ * 32 == 0).  Gate and up scales may have different group counts.  Otherwise
+ * two linears into the workspace and an elementwise launch; size the workspace
+ * with gi_w4a16_gated_mlp_workspace_bytes.                                  */
 size_t gi_w4a16_gated_mlp_workspace_bytes(int M, int K, int N, int group_size);
 int gi_w4a16_gated_mlp(const void* A, int a_dtype,
                        const int32_t* gate_packed, const void* gate_scales, int gate_groups,

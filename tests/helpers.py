@@ -7,8 +7,8 @@ import torch
 from oracle import moe_oracle as O
 
 # Tolerance gate for bf16 outputs against the float64 oracle.
-#   * rel-L2 <= 1e-2: the bound of BASELINE.json's north_star, literally.
-#   * elementwise |got - ref| <= 2e-2 + 2^-7 |ref|: the north-star max-abs 2e-2
+#   * rel-L2 <= 1e-2: the bound that bf16 parity is judged by, literally.
+#   * elementwise |got - ref| <= 2e-2 + 2^-7 |ref|: its max-abs bound 2e-2
 #     made scale-aware.  A literal max-abs of 2e-2 is below the bf16 spacing of
 #     outputs this large (|out| reaches 50-85, spacing 0.25-0.5); 2^-7 |ref| is
 #     two half-ulps of bf16.
@@ -43,7 +43,7 @@ def assert_close_rms(got: torch.Tensor, ref64: np.ndarray, what: str = "",
     (its float64 value within fp32 error of a rounding midpoint) move an output
     by amounts that scale with the terms, not with the output, so the
     elementwise 2e-2 + 2^-7|ref| bound does not apply.  Instead: rel-L2 <= 1e-2
-    (literally) and max |got - ref| <= max_over_rms * RMS(ref)
+    (that bound, literally) and max |got - ref| <= max_over_rms * RMS(ref)
     (the max-abs bound in units of the output's own size)."""
     g = np64(got)
     stats = O.error_stats(g, ref64)
@@ -83,7 +83,7 @@ def assert_dtype_close(got: torch.Tensor, ref64: np.ndarray, dtype: str, what: s
     """The tolerance gate for outputs in the activation dtype of a call.
 
     bf16: assert_bf16_close.  fp16: rel-L2 <= 1e-2 and every element within
-    2e-2 + 2^-10 |ref| (the north-star max-abs plus one fp16 ulp; fp16 keeps 3
+    2e-2 + 2^-10 |ref| (that max-abs bound plus one fp16 ulp; fp16 keeps 3
     more mantissa bits than bf16).  fp32 (nothing is rounded but the float32
     sums): rel-L2 <= 2e-5 and max |got - ref| <= 1e-4 * RMS(ref)."""
     if dtype == "bf16":
@@ -117,7 +117,7 @@ def kernels_of(call) -> list:
     return names
 
 
-# Error statistics of the BASELINE configs' parity tests, by config name;
+# Error statistics of the parity tests of the benchmark workloads, by name;
 # tests/conftest.py writes them to the JSON file named by GI_PARITY_STATS
 # at the end of the session (when that variable is set).
 PARITY_RECORD: dict = {}

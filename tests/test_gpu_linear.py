@@ -13,7 +13,7 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("m,k,n,gs", [
-    (1, 2816, 2816, 128),    # BASELINE config 0 shape
+    (1, 2816, 2816, 128),    # the benchmark's linear
     (5, 2816, 2112, 64),     # reference sanitizer test shape (M=5)
     (16, 2816, 2112, 64),    # M > 8 (reference's coalesced path)
     (8, 256, 1000, 64),      # test-small lm_head (vocab 1000)
@@ -62,7 +62,7 @@ def test_w4a16_reference_floor_groups_drop_tail():
 
 
 def test_lm_head_softcap_column_subset():
-    """BASELINE config 4 shape (M=6, K=2816, N=262144, gs=128): every output is
+    """The benchmark's lm_head (M=6, K=2816, N=262144, gs=128): every output is
     computed on the GPU; the float64 oracle checks 2048 random columns."""
     m, k, n, gs = 6, 2816, 262144, 128
     g = torch.Generator(device=DEV)
