@@ -85,6 +85,10 @@ int* device_error_flag(bool allocate, hipStream_t stream) {
   return (int*)d;
 }
 
+void ensure_device_error_flags(hipStream_t stream) {
+  if (!flags_host(false)) (void)device_error_flag(true, stream);
+}
+
 int read_device_error_flags(int device, int clear) {
   if (device < 0 || device >= 64) return fail(GI_ERR_INVALID_ARG, "device_error_flags: device index out of range");
   int* h = flags_host(true);

@@ -25,6 +25,9 @@ int device_cu_count();
 // call with allocate = true whose stream is not capturing a graph;
 // allocate = false only returns them once they exist.
 int* device_error_flag(bool allocate, hipStream_t stream);
+// Allocates the flags, on the same condition, for a launch that does not write
+// them (later launches under capture find them).
+void ensure_device_error_flags(hipStream_t stream);
 int read_device_error_flags(int device, int clear);
 
 // ---- fused MoE --------------------------------------------------------------

@@ -1168,6 +1168,7 @@ int launch_fused_moe(const MoeHostArgs& h) {
   if (((uintptr_t)h.workspace) % kAlign)
     return fail(GI_ERR_WORKSPACE, "fused MoE: workspace must be 256-byte aligned");
   if (moe_prefill_supported(h)) {
+    ensure_device_error_flags(h.stream);  // as the launches of 8 rows do
     const size_t base = prefill_base(h.H, h.I);
     const WsLayout L = ws_layout(1, h.H, h.I, kTaskCols);
     return launch_moe_prefill(h, (char*)h.workspace + base, h.workspace_bytes - base,
